@@ -482,9 +482,9 @@ int trk_last_timing(const trk_ctx *c, double *transport_s, double *total_s, int6
 int trk_set_profiling(trk_ctx *c, int on)
 {
     if (!c) return TRK_ERR_ARG;
-    if (on && !c->pe[0]) {
-        if (hipEventCreate(&c->pe[0]) != hipSuccess || hipEventCreate(&c->pe[1]) != hipSuccess)
-            return set_error(c, TRK_ERR_DEVICE, "hipEventCreate failed");
+    if (on) {
+        for (hipEvent_t &e : c->pe)
+            if (!e && hipEventCreate(&e) != hipSuccess) return set_error(c, TRK_ERR_DEVICE, "hipEventCreate failed");
     }
     c->prof = on != 0;
     if (on) {

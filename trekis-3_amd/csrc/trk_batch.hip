@@ -76,6 +76,7 @@ struct trk_batch {
     trk::McDev mc[trk::kMaxGroups][2];
     int capacity = 0;
     int block = 768, round_events = 512;
+    bool ion_deep = true;          // ions may take more than round_events collisions in a round
     int64_t blocks = 0;
     size_t lds_bytes = 0;
     bool all_staged = false;
@@ -161,6 +162,7 @@ __global__ void k_batch_reset(BatchCtl *ctl, int n_groups, unsigned long long de
         }
         gc->n_in[K_ION] = n_ions[g];
         gc->cursor = 0;
+        gc->ion_cursor = 0;
         gc->cur = 0;
         gc->overflow = 0;
     }
@@ -299,6 +301,7 @@ static void batch_descriptors(trk_batch *b)
             }
             d.out_cnt = &gr.gctl->out_cnt[1 - par][0];
             d.cursor = &gr.gctl->cursor;
+            d.ion_cursor = &gr.gctl->ion_cursor;
             d.overflow = b->d_overflow;
             d.counters = b->d_counters;
             d.T = gr.T;
@@ -311,6 +314,14 @@ static void batch_descriptors(trk_batch *b)
             d.ions = b->d_ions;
             d.plane_of = b->d_plane_of;
             d.round_events = b->round_events;
+            // an ion runs to its end in one round while the pairs of all the
+            // group's ions take a quarter of its lists at most
+            double pairs = 0.0;
+            for (int i : gr.members) {
+                const double lam = b->impacts[i]->ts.shi_path0;
+                pairs += (lam > 0.0) ? h.m.Layer / lam : 1e4;
+            }
+            d.ion_events = ion_round_events(pairs, (int)gr.members.size(), gr.cap[K_EL], b->round_events, b->ion_deep);
             d.gctl = gr.gctl;
             size_t bytes = 0;
             const size_t limit = ((size_t)b->max_lds - 256) / sizeof(double);
@@ -413,6 +424,13 @@ static int batch_launch(trk_batch *b, uint64_t seed, int64_t first_iter, trk_tal
         GroupCtl gc{};
         BHIP(hipMemcpy(&gc, b->groups[g].gctl, sizeof gc, hipMemcpyDeviceToHost));
         if (gc.overflow) ovf |= kFlagPairs;
+    }
+    if (ovf && b->ion_deep) {
+        // the same impacts with their ions held to the round budget, which
+        // spreads the pairs over the rounds
+        b->ion_deep = false;
+        batch_descriptors(b);
+        return batch_launch(b, seed, first_iter, outs);
     }
     if (ovf) return berr(b, TRK_ERR_CAPACITY, "particle list capacity %d exceeded (flags %d)", b->capacity, ovf);
     unsigned long long ctr[16];

@@ -69,7 +69,7 @@ struct trk_ctx {
     bool prof = false;
     double k_ms[2] = {0.0, 0.0};
     int64_t k_launches[2] = {0, 0};
-    hipEvent_t pe[2] = {nullptr, nullptr};
+    hipEvent_t pe[4] = {nullptr, nullptr, nullptr, nullptr};   // transport, ions
     // tracing
     double *trace_host = nullptr;
     int64_t trace_cap = 0;

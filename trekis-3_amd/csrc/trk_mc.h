@@ -63,7 +63,7 @@ struct GroupCtl {
     int cursor;
     int cur;
     int overflow;
-    int pad_;
+    int ion_cursor;
 };
 
 // Control of a batch launch (device memory): the grid barrier, the round
@@ -148,6 +148,9 @@ struct McDev {
     const double *beb_Ek;
     // DSF elastic scattering (kind_of_EMFP = 2) of electrons [0] and holes [1]
     DsfDev dsf[2];
+    // the next ion of the current round and the collisions an ion may take in it
+    int *ion_cursor;
+    int ion_events;
 };
 
 enum { EV_SHI = 0, EV_E_INEL, EV_E_EL, EV_H_INEL, EV_H_EL, EV_AUGER, EV_RAD, EV_PHOT };
@@ -160,7 +163,7 @@ constexpr uint32_t kMaxEvents = 1u << 22;
 
 enum { K_EL = 0, K_HO = 1, K_PH = 2, K_ION = 3 };
 
-enum { C_E_EL = 0, C_E_INEL, C_H_EL, C_H_INEL, C_DEEP, C_PHOT, C_ION, C_COUNT };
+enum { C_E_EL = 0, C_E_INEL, C_H_EL, C_H_INEL, C_DEEP, C_PHOT, C_COUNT };
 
 // A wave runs a category of events only when at least this many of its lanes
 // want it (or when it is the most wanted one); the other lanes wait with
@@ -183,11 +186,15 @@ extern __shared__ double lds_tab[];
 constexpr int kTransportBlockFp64 = 768;
 constexpr int kTransportBlockMx = 768;
 
+// Workgroup of the ion kernel: 8 waves, each with one ion, 2 per SIMD.
+constexpr int kIonBlock = 512;
+
 // The event code is compiled twice, into namespaces fp64 (deterministic
 // FP64, replays the oracle bit for bit) and mx (mixed precision); these are
 // the kernels the host driver launches from each.
 #define TRK_MC_KERNELS                                                          \
     template <bool kAll, bool kGeneral> __global__ void k_transport(McDev din); \
+    template <bool kAll> __global__ void k_ions(McDev din, int waves);       \
     __global__ void k_ion_init(McDev d, int nb, uint32_t first_iter);        \
     __global__ void k_shi_consts(IonDev iv, const double *Ip, int nsh, int *sd_M, double *sd_c); \
     __global__ void k_shi_buckets(IonDev iv, int nsh, const int *sd_M, const double *sd_c, int *sd_bk); \
@@ -205,6 +212,18 @@ hipError_t launch_shi_consts(const trk_ctx *c, const IonDev &iv, bool mixed, hip
 void fill_mcdev(const trk_ctx *c, McDev &d);
 // LDS layout of the staged tables (trk_mc.hip); true when all are staged.
 bool plan_lds(McDev &d, int Nt, int NR, int n_dos, int nsh, size_t limit_doubles, size_t *bytes);
+// Collisions an ion may take in one round: all of them while the pairs they
+// make (expected number) take a quarter of the lists at most, else as many as
+// do, and never fewer than the other particles' budget (deep = false: just
+// that).  A run whose lists overflow is repeated with deep = false, so that
+// no list has to be longer than with one budget for all.
+static inline int ion_round_events(double pairs, int n_ions, int cap, int round_events, bool deep)
+{
+    if (!deep) return round_events;
+    if (pairs <= 0.25 * cap) return 1 << 30;
+    const int n = (int)(0.25 * cap / n_ions);
+    return n > round_events ? n : round_events;
+}
 // BEB shells or the Delta-CDF model: the transport kernel's general instantiation
 bool uses_general_kernel(const HostMat &h);
 // One tally plane converted and added into the caller's Out_* arrays (trk_mc.hip).

@@ -565,12 +565,18 @@ int finish_tallies_host(trk_ctx *c, const Tally &T, int plane_index, const doubl
 // ionisations is at most a few hundred long.
 constexpr int kMaxGenerations = 1 << 16;
 
-// Iterations per batch: the ion's expected ionisations over the layer times
-// the pairs each makes must fit one generation's lists.
-static int64_t batch_size(const trk_ctx *c, int cap, int64_t nmc)
+// The ion's expected ionisations over the layer.
+static double ion_collisions(const trk_ctx *c)
 {
     const double lam = c->ts.shi_path0;
-    const double est_pairs = (lam > 0.0) ? c->hm.m.Layer / lam : 1e4;
+    return (lam > 0.0) ? c->hm.m.Layer / lam : 1e4;
+}
+
+// Iterations per batch: the ion's expected ionisations times the pairs each
+// makes must fit one generation's lists.
+static int64_t batch_size(const trk_ctx *c, int cap, int64_t nmc)
+{
+    const double est_pairs = ion_collisions(c);
     int64_t B = (c->hm.o.batch > 0) ? c->hm.o.batch : (int64_t)((double)cap / (3.0 * est_pairs + 64.0));
     if (B < 1) B = 1;
     if (B > nmc) B = nmc;
@@ -672,9 +678,11 @@ static const void *transport_kernel(bool mixed, bool all, bool general)
 // The run itself on buffers the caller of this function provides in s (and
 // na, for a run without allocation: the tallies are then finished on the
 // device instead of the host).
-static int run_core(trk_ctx *c, McState *s, int64_t nmc, uint64_t seed, int64_t first_iter, const double *Out_R,
-                    const double *Out_V, int NR, trk_tallies *out, int64_t B, bool want_spec,
-                    const NoAllocBufs *nab = nullptr)
+// deep: the ions may run further in a round than the other particles; *lists_full
+// is set when a list overflowed with that in use.
+static int run_rounds(trk_ctx *c, McState *s, int64_t nmc, uint64_t seed, int64_t first_iter, const double *Out_R,
+                      const double *Out_V, int NR, trk_tallies *out, int64_t B, bool want_spec, const NoAllocBufs *nab,
+                      bool deep, bool *lists_full)
 {
     auto tstart = std::chrono::steady_clock::now();
     const bool mixed = c->hm.o.precision == 1;   // FP32 elementary functions in the event code
@@ -735,6 +743,9 @@ static int run_core(trk_ctx *c, McState *s, int64_t nmc, uint64_t seed, int64_t 
         d.trace = s->d_trace; d.trace_n = s->d_trace_n; d.trace_cap = c->trace_cap;
     }
     for (int k = 0; k < 4; ++k) d.cap[k] = s->cap[k];
+    d.cursor = s->d_counts + 8;
+    d.ion_cursor = s->d_counts + 9;
+    d.ion_events = ion_round_events((double)B * ion_collisions(c), (int)B, s->cap[K_EL], (int)kRoundEvents, deep);
 
     // per-iteration normalised tallies, when the caller asks for any of them
     const int ND = h.m.n_dos;
@@ -776,6 +787,11 @@ static int run_core(trk_ctx *c, McState *s, int64_t nmc, uint64_t seed, int64_t 
                                                           s->lds_bytes));
         if (per_cu < 1) per_cu = 1;
         s->max_blocks = (int64_t)per_cu * s->ncu;
+        if (s->lds_bytes > 65536) {
+            const void *ki = mixed ? (all ? (const void *)mx::k_ions<true> : (const void *)mx::k_ions<false>)
+                                   : (all ? (const void *)fp64::k_ions<true> : (const void *)fp64::k_ions<false>);
+            HIPC(hipFuncSetAttribute(ki, hipFuncAttributeMaxDynamicSharedMemorySize, (int)s->lds_bytes));
+        }
     }
 
     double transport_s = 0.0;
@@ -804,80 +820,101 @@ static int run_core(trk_ctx *c, McState *s, int64_t nmc, uint64_t seed, int64_t 
         }
         for (int k = 0; k < 4; ++k) d.in[k] = s->L[cur][k];
         if (s->ev0) HIPC(hipEventRecord(s->ev0, st));
-        if (c->prof) HIPC(hipEventRecord(c->pe[0], st));
+        if (c->prof) HIPC(hipEventRecord(c->pe[2], st));
         if (mixed) mx::k_ion_init<<<(nb + 63) / 64, 64, 0, st>>>(d, nb, (uint32_t)(first_iter + b0));
         else fp64::k_ion_init<<<(nb + 63) / 64, 64, 0, st>>>(d, nb, (uint32_t)(first_iter + b0));
         HIPC(hipGetLastError());
-        if (c->prof) HIPC(hipEventRecord(c->pe[1], st));
+        if (c->prof) HIPC(hipEventRecord(c->pe[3], st));
         launches++;
-        int pending = 0;          // kernel whose events are still to be read
+        bool pending[2] = {true, false};          // kernels (SHI, transport) whose events are still to be read
         int nin[4] = {0, 0, 0, nb};
         for (;;) {
             if (rounds > 0) {
                 HIPC(hipMemcpyAsync(hc, s->d_counts + 4 * cur, 4 * sizeof(int), hipMemcpyDeviceToHost, st));
             }
             HIPC(hipStreamSynchronize(st));
-            if (c->prof && pending >= 0) {
+            for (int k = 0; c->prof && k < 2; ++k) {
+                if (!pending[k]) continue;
                 float kms = 0.f;
-                HIPC(hipEventElapsedTime(&kms, c->pe[0], c->pe[1]));
-                c->k_ms[pending] += kms;
-                c->k_launches[pending]++;
-                pending = -1;
+                hipEvent_t *pe = c->pe + (k == TRK_K_SHI ? 2 : 0);
+                HIPC(hipEventElapsedTime(&kms, pe[0], pe[1]));
+                c->k_ms[k] += kms;
+                c->k_launches[k]++;
+                pending[k] = false;
             }
             int ovf = 0;
             HIPC(hipMemcpy(&ovf, s->d_overflow, sizeof(int), hipMemcpyDeviceToHost));
             if (ovf & kFlagNaN) return set_error(c, TRK_ERR_NUMERIC, "a particle state became NaN (iterations %lld..%lld)",
                                                   (long long)(first_iter + b0), (long long)(first_iter + b0 + nb - 1));
             if (ovf & kFlagEvents) return set_error(c, TRK_ERR_CAPACITY, "a particle exceeded %u events", kMaxEvents);
-            if (ovf)
+            if (ovf) {
+                *lists_full = d.ion_events > (int)kRoundEvents;
                 return set_error(c, TRK_ERR_CAPACITY,
                                  "particle list capacity exceeded (flags %d, round %d, batch %lld; capacities e %d h %d p %d ion %d)",
                                  ovf, rounds, (long long)B, s->cap[0], s->cap[1], s->cap[2], s->cap[3]);
+            }
             if (++rounds > kMaxGenerations) return set_error(c, TRK_ERR_CAPACITY, "more than %d transport rounds", kMaxGenerations);
             if (rounds > 1)
                 for (int k = 0; k < 4; ++k) nin[k] = hc[k] < s->cap[k] ? hc[k] : s->cap[k];
             if (verbose)
                 fprintf(stderr, "[trk] batch %lld round %d: electrons %d holes %d photons %d ions %d\n",
                         (long long)b0, rounds, nin[0], nin[1], nin[2], nin[3]);
-            int64_t nthr = (int64_t)nin[0] + nin[1] + nin[2] + nin[3];
-            if (nthr == 0) break;
+            const int64_t nthr = (int64_t)nin[0] + nin[1] + nin[2];
+            if (nthr == 0 && nin[K_ION] == 0) break;
             int nxt = 1 - cur;
             HIPC(hipMemsetAsync(s->d_counts + 4 * nxt, 0, 4 * sizeof(int), st));
             for (int k = 0; k < 4; ++k) { d.in[k] = s->L[cur][k]; d.out[k] = s->L[nxt][k]; d.n_in[k] = nin[k]; }
             d.out_cnt = s->d_counts + 4 * nxt;
-            const int tb = mixed ? kTransportBlockMx : kTransportBlockFp64;
-            int64_t nblk = (nthr + tb - 1) / tb;
-            int tbl = tb;             // threads per workgroup of this launch
-            if (nblk < s->max_blocks) {
-                // few particles (the ions' first round, the last rounds):
-                // spread them over the resident workgroups, one or a few
-                // waves each, rather than full workgroups on a few CUs (the
-                // kernel stages its tables with blockDim.x threads)
-                const int64_t waves = (nthr + 63) / 64;
-                const int64_t w = (waves + s->max_blocks - 1) / s->max_blocks;
-                tbl = (int)(64 * w);
-                nblk = (nthr + tbl - 1) / tbl;
-            }
-            if (nblk > s->max_blocks) nblk = s->max_blocks;
-            d.cursor = s->d_counts + 8;
-            HIPC(hipMemsetAsync(d.cursor, 0, sizeof(int), st));
-            if (c->prof) HIPC(hipEventRecord(c->pe[0], st));
-            const unsigned g = (unsigned)nblk;
+            HIPC(hipMemsetAsync(d.cursor, 0, 2 * sizeof(int), st));
             const size_t lds = s->lds_bytes;
-            if (general) {
-                if (mixed && s->all_staged) mx::k_transport<true, true><<<g, tbl, lds, st>>>(d);
-                else if (mixed) mx::k_transport<false, true><<<g, tbl, lds, st>>>(d);
-                else if (s->all_staged) fp64::k_transport<true, true><<<g, tbl, lds, st>>>(d);
-                else fp64::k_transport<false, true><<<g, tbl, lds, st>>>(d);
-            } else {
-                if (mixed && s->all_staged) mx::k_transport<true, false><<<g, tbl, lds, st>>>(d);
-                else if (mixed) mx::k_transport<false, false><<<g, tbl, lds, st>>>(d);
-                else if (s->all_staged) fp64::k_transport<true, false><<<g, tbl, lds, st>>>(d);
-                else fp64::k_transport<false, false><<<g, tbl, lds, st>>>(d);
+            if (nin[K_ION] > 0) {
+                // one wave per ion: one per CU while there are few, up to the
+                // workgroup's eight
+                const int64_t per = (nin[K_ION] + s->ncu - 1) / s->ncu;
+                const int waves = (int)(per < kIonBlock / 64 ? per : kIonBlock / 64);
+                const int64_t need = (nin[K_ION] + waves - 1) / waves;
+                const unsigned gi = (unsigned)(need < s->ncu ? need : s->ncu);
+                if (c->prof) HIPC(hipEventRecord(c->pe[2], st));
+                if (mixed && s->all_staged) mx::k_ions<true><<<gi, kIonBlock, lds, st>>>(d, waves);
+                else if (mixed) mx::k_ions<false><<<gi, kIonBlock, lds, st>>>(d, waves);
+                else if (s->all_staged) fp64::k_ions<true><<<gi, kIonBlock, lds, st>>>(d, waves);
+                else fp64::k_ions<false><<<gi, kIonBlock, lds, st>>>(d, waves);
+                HIPC(hipGetLastError());
+                if (c->prof) { HIPC(hipEventRecord(c->pe[3], st)); pending[TRK_K_SHI] = true; }
+                launches++;
             }
-            HIPC(hipGetLastError());
-            if (c->prof) { HIPC(hipEventRecord(c->pe[1], st)); pending = 1; }
-            launches++;
+            if (nthr > 0) {
+                const int tb = mixed ? kTransportBlockMx : kTransportBlockFp64;
+                int64_t nblk = (nthr + tb - 1) / tb;
+                int tbl = tb;             // threads per workgroup of this launch
+                if (nblk < s->max_blocks) {
+                    // few particles (the last rounds): spread them over the
+                    // resident workgroups, one or a few waves each, rather
+                    // than full workgroups on a few CUs (the kernel stages
+                    // its tables with blockDim.x threads)
+                    const int64_t waves = (nthr + 63) / 64;
+                    const int64_t w = (waves + s->max_blocks - 1) / s->max_blocks;
+                    tbl = (int)(64 * w);
+                    nblk = (nthr + tbl - 1) / tbl;
+                }
+                if (nblk > s->max_blocks) nblk = s->max_blocks;
+                if (c->prof) HIPC(hipEventRecord(c->pe[0], st));
+                const unsigned g = (unsigned)nblk;
+                if (general) {
+                    if (mixed && s->all_staged) mx::k_transport<true, true><<<g, tbl, lds, st>>>(d);
+                    else if (mixed) mx::k_transport<false, true><<<g, tbl, lds, st>>>(d);
+                    else if (s->all_staged) fp64::k_transport<true, true><<<g, tbl, lds, st>>>(d);
+                    else fp64::k_transport<false, true><<<g, tbl, lds, st>>>(d);
+                } else {
+                    if (mixed && s->all_staged) mx::k_transport<true, false><<<g, tbl, lds, st>>>(d);
+                    else if (mixed) mx::k_transport<false, false><<<g, tbl, lds, st>>>(d);
+                    else if (s->all_staged) fp64::k_transport<true, false><<<g, tbl, lds, st>>>(d);
+                    else fp64::k_transport<false, false><<<g, tbl, lds, st>>>(d);
+                }
+                HIPC(hipGetLastError());
+                if (c->prof) { HIPC(hipEventRecord(c->pe[1], st)); pending[TRK_K_TRANSPORT] = true; }
+                launches++;
+            }
             cur = nxt;
         }
         if (want_spec) {
@@ -977,6 +1014,19 @@ static int run_core(trk_ctx *c, McState *s, int64_t nmc, uint64_t seed, int64_t 
     c->last_total_s = std::chrono::duration<double>(std::chrono::steady_clock::now() - tstart).count();
     c->last_launches = launches;
     return 0;
+}
+
+// run_rounds, and once more with the ions held to the particles' round budget
+// if a list overflowed while they ran further (nothing has been added to the
+// caller's tallies by then).
+static int run_core(trk_ctx *c, McState *s, int64_t nmc, uint64_t seed, int64_t first_iter, const double *Out_R,
+                    const double *Out_V, int NR, trk_tallies *out, int64_t B, bool want_spec,
+                    const NoAllocBufs *nab = nullptr)
+{
+    bool full = false;
+    const int rc = run_rounds(c, s, nmc, seed, first_iter, Out_R, Out_V, NR, out, B, want_spec, nab, true, &full);
+    if (!rc || !full) return rc;
+    return run_rounds(c, s, nmc, seed, first_iter, Out_R, Out_V, NR, out, B, want_spec, nab, false, &full);
 }
 
 // do_Monte_Carlo on buffers this context allocates on its first run and

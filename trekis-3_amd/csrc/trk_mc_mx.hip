@@ -11,6 +11,8 @@ template __global__ void k_transport<true, false>(McDev din);
 template __global__ void k_transport<false, false>(McDev din);
 template __global__ void k_transport<true, true>(McDev din);
 template __global__ void k_transport<false, true>(McDev din);
+template __global__ void k_ions<true>(McDev din, int waves);
+template __global__ void k_ions<false>(McDev din, int waves);
 template __global__ void k_batch<true>(BatchCtl *ctl, int n_groups);
 template __global__ void k_batch<false>(BatchCtl *ctl, int n_groups);
 }  // namespace mx
