@@ -314,6 +314,7 @@ static void batch_descriptors(trk_batch *b)
             d.ions = b->d_ions;
             d.plane_of = b->d_plane_of;
             d.round_events = b->round_events;
+            d.lane_cap = 64;
             // an ion runs to its end in one round while the pairs of all the
             // group's ions take a quarter of its lists at most
             double pairs = 0.0;

@@ -40,7 +40,7 @@ struct Spec {
 };
 
 // tables staged in each transport workgroup's LDS (see stage_tables)
-constexpr int kStaged = 26;
+constexpr int kStaged = 34;
 
 // The ion of one impact: its parameters and its own tables (SHI_MFP, the
 // fused SHI_path, diff_SHI_MFP at its initial energy and the mixed path's
@@ -151,6 +151,8 @@ struct McDev {
     // the next ion of the current round and the collisions an ion may take in it
     int *ion_cursor;
     int ion_events;
+    // lanes of a wave that take particles (run_items)
+    int lane_cap;
 };
 
 enum { EV_SHI = 0, EV_E_INEL, EV_E_EL, EV_H_INEL, EV_H_EL, EV_AUGER, EV_RAD, EV_PHOT };
@@ -172,6 +174,11 @@ enum { C_E_EL = 0, C_E_INEL, C_H_EL, C_H_INEL, C_DEEP, C_PHOT, C_COUNT };
 constexpr int kBatchLanes = 16;
 constexpr int kMaxWait = 16;
 
+// A moving particle's flight over more nodes than this is tallied by its whole
+// wave.  One lane needs about 2800 cycles a node (shared with the wave's other
+// long flights), the wave about 2000 cycles a flight.
+constexpr int kWaveNodes = 3;
+
 // Events one particle may take in one round.  A particle with more left is
 // written to the next round's list; this bounds the tail of every launch by
 // the cost of kRoundEvents events instead of the longest history.
@@ -179,12 +186,22 @@ constexpr uint32_t kRoundEvents = 512;
 
 extern __shared__ double lds_tab[];
 
+// The sources a path's kernels are spread over (TRK_PART): the transport of
+// single runs with its set-up kernels, the ions and the general transfers, and
+// the batch kernels.
+#define TRK_PART_RUN 0
+#define TRK_PART_GENERAL 1
+#define TRK_PART_BATCH 2
+
 // Transport workgroup of each path: one per CU (the staged tables fill most
 // of the LDS), 12 waves, 3 per SIMD (168 VGPRs).  At 16 waves the mixed
 // path would have to spill to scratch, which costs more than the fourth
 // wave gains.
 constexpr int kTransportBlockFp64 = 768;
 constexpr int kTransportBlockMx = 768;
+
+// Waves per workgroup (one per SIMD) of a round with few particles.
+constexpr int kSparseWaves = 4;
 
 // Workgroup of the ion kernel: 8 waves, each with one ion, 2 per SIMD.
 constexpr int kIonBlock = 512;

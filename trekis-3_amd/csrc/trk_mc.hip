@@ -591,12 +591,14 @@ bool plan_lds(McDev &d, int Nt, int NR, int n_dos, int nsh, size_t limit, size_t
     const int nsz[kStaged] = {d.nE, d.nE, d.nE, d.nE, d.nEel, d.nEel, d.nEel, d.nEel,
                               d.nH, d.nH, d.nH, d.nH, d.nHel, d.nHel, d.nHel, d.nHel,
                               NR, Nt, n_dos, n_dos, n_dos, n_dos, nsh * d.nE, nsh * d.nH,
-                              nsh * d.nE, nsh * d.nH};
+                              nsh * d.nE, nsh * d.nH, nsh, nsh, nsh, nsh,
+                              d.m.n_atoms, d.m.n_atoms, d.m.n_atoms, d.m.n_atoms};
     const bool present[kStaged] = {true, true, d.lnE != nullptr, d.ln_el_imfp != nullptr, true, true,
                                    d.lnEel != nullptr, d.ln_Lel != nullptr, true, true, d.lnEH != nullptr,
                                    d.ln_hole_imfp != nullptr, true, true, d.lnEHel != nullptr,
                                    d.ln_LHel != nullptr, true, true, true, true, true, true, true, true,
-                                   d.ln_Lsh != nullptr, d.ln_LHsh != nullptr};
+                                   d.ln_Lsh != nullptr, d.ln_LHsh != nullptr, true, true, true, true,
+                                   true, true, true, true};
     size_t off = 0;
     bool all = true;
     for (int a = 0; a < kStaged; ++a) {
@@ -887,15 +889,17 @@ static int run_rounds(trk_ctx *c, McState *s, int64_t nmc, uint64_t seed, int64_
                 const int tb = mixed ? kTransportBlockMx : kTransportBlockFp64;
                 int64_t nblk = (nthr + tb - 1) / tb;
                 int tbl = tb;             // threads per workgroup of this launch
-                if (nblk < s->max_blocks) {
-                    // few particles (the last rounds): spread them over the
-                    // resident workgroups, one or a few waves each, rather
-                    // than full workgroups on a few CUs (the kernel stages
-                    // its tables with blockDim.x threads)
-                    const int64_t waves = (nthr + 63) / 64;
-                    const int64_t w = (waves + s->max_blocks - 1) / s->max_blocks;
-                    tbl = (int)(64 * w);
-                    nblk = (nthr + tbl - 1) / tbl;
+                d.lane_cap = 64;
+                if (nthr < 64 * kSparseWaves * s->max_blocks) {
+                    // few particles (the last rounds of a large run, all of
+                    // a small one): as many waves as there are SIMDs, with as
+                    // few particles each as that gives; a wave runs each
+                    // category its particles want in turn, so a lone history
+                    // goes faster the fewer share its wave
+                    tbl = 64 * kSparseWaves;
+                    d.lane_cap = (int)((nthr + kSparseWaves * s->max_blocks - 1) / (kSparseWaves * s->max_blocks));
+                    const int64_t per = (int64_t)kSparseWaves * d.lane_cap;
+                    nblk = (nthr + per - 1) / per;
                 }
                 if (nblk > s->max_blocks) nblk = s->max_blocks;
                 if (c->prof) HIPC(hipEventRecord(c->pe[0], st));
