@@ -26,6 +26,11 @@
  *         |x| > 1 uses pi/2 - atan(1/x).
  *   acos  acos x = 2 atan(sqrt((1-x)/(1+x))).
  *   pow   exp(y log x) for x > 0.
+ * Special arguments (NaN, infinities, out of range) are replaced by a harmless
+ * one on the way in and their result is put in on the way out, without
+ * branches: on a GPU several evaluations in a row then form one block of
+ * straight code and overlap, where a wave's dependent FP64 operations leave
+ * most of the issue slots of a lone history empty.
  * Accuracy is a few ulp (checked against mpmath in the tests); the point is
  * reproducibility, not correct rounding.
  */
@@ -67,11 +72,10 @@ TRK_FN double trk_exp(double x)
     const double INV_LN2 = 0x1.71547652b82fep+0;
     const double LN2_HI = 0x1.62e42fee00000p-1;
     const double LN2_LO = 0x1.a39ef35793c76p-33;
-    if (x != x) return x;
-    if (x > 709.782712893384) return TRK_INF;
-    if (x < -745.1332191019412) return 0.0;
-    double kd = trk_rint(x * INV_LN2);
-    double r = (x - kd * LN2_HI) - kd * LN2_LO;
+    const int over = x > 709.782712893384, under = x < -745.1332191019412, nan = x != x;
+    const double xc = (over || under || nan) ? 0.0 : x;
+    double kd = trk_rint(xc * INV_LN2);
+    double r = (xc - kd * LN2_HI) - kd * LN2_LO;
     double p = 0x1.6827863b97d97p-53;          /* 1/18! */
     p = 0x1.952c77030ad4ap-49 + r * p;         /* 1/17! */
     p = 0x1.ae7f3e733b81fp-45 + r * p;         /* 1/16! */
@@ -94,7 +98,10 @@ TRK_FN double trk_exp(double x)
     int k = (int)kd;
     int k1 = k / 2;
     int k2 = k - k1;
-    return (e * trk_pow2i(k1)) * trk_pow2i(k2);
+    double v = (e * trk_pow2i(k1)) * trk_pow2i(k2);
+    v = over ? TRK_INF : v;
+    v = under ? 0.0 : v;
+    return nan ? x : v;
 }
 
 /* --- log ------------------------------------------------------------------ */
@@ -103,20 +110,15 @@ TRK_FN double trk_log(double x)
     const double LN2_HI = 0x1.62e42fee00000p-1;
     const double LN2_LO = 0x1.a39ef35793c76p-33;
     const double SQRT2 = 0x1.6a09e667f3bcdp+0;
-    if (x != x) return x;
-    if (x < 0.0) return TRK_NAN;
-    if (x == 0.0) return -TRK_INF;
-    if (x == TRK_INF) return x;
-    int e = 0;
-    uint64_t u = trk_d2u(x);
-    if ((u >> 52) == 0) {                      /* subnormal */
-        x = x * 0x1.0p+54;
-        u = trk_d2u(x);
-        e = -54;
-    }
-    e += (int)(u >> 52) - 1023;
+    const int plain = x > 0.0 && x < TRK_INF;
+    const double xp = plain ? x : 1.0;
+    const int sub = (trk_d2u(xp) >> 52) == 0;  /* subnormal */
+    const uint64_t u = trk_d2u(sub ? xp * 0x1.0p+54 : xp);
+    int e = (sub ? -54 : 0) + ((int)(u >> 52) - 1023);
     double m = trk_u2d((u & 0x000FFFFFFFFFFFFFull) | 0x3FF0000000000000ull);
-    if (m > SQRT2) { m = m * 0.5; e += 1; }
+    const int half = m > SQRT2;
+    m = half ? m * 0.5 : m;
+    e += half;
     double f = m - 1.0;
     double s = f / (2.0 + f);
     double z = s * s;
@@ -136,7 +138,10 @@ TRK_FN double trk_log(double x)
     double s2 = 2.0 * s;
     double logm = s2 + s2 * (z * R);
     double ed = (double)e;
-    return ed * LN2_HI + (ed * LN2_LO + logm);
+    double v = ed * LN2_HI + (ed * LN2_LO + logm);
+    double w = (x == 0.0) ? -TRK_INF : x;      /* NaN and +infinity are their own logarithms */
+    w = (x < 0.0) ? TRK_NAN : w;
+    return plain ? v : w;
 }
 
 /* --- sin / cos -------------------------------------------------------------- */
@@ -187,36 +192,40 @@ TRK_FN double trk_reduce_pio2(double x, int *q)
  * would run every path anyway. */
 TRK_FN double trk_sin(double x)
 {
-    if (x != x || trk_fabs(x) == TRK_INF) return TRK_NAN;
+    const int bad = !(trk_fabs(x) < TRK_INF);
     int q;
-    double r = trk_reduce_pio2(x, &q);
+    double r = trk_reduce_pio2(bad ? 0.0 : x, &q);
     double sp = trk_sin_poly(r), cp = trk_cos_poly(r);
     double v = (q & 1) ? cp : sp;
-    return (q & 2) ? -v : v;
+    v = (q & 2) ? -v : v;
+    return bad ? TRK_NAN : v;
 }
 
 TRK_FN double trk_cos(double x)
 {
-    if (x != x || trk_fabs(x) == TRK_INF) return TRK_NAN;
+    const int bad = !(trk_fabs(x) < TRK_INF);
     int q;
-    double r = trk_reduce_pio2(x, &q);
+    double r = trk_reduce_pio2(bad ? 0.0 : x, &q);
     double sp = trk_sin_poly(r), cp = trk_cos_poly(r);
     double v = (q & 1) ? sp : cp;
-    return ((q + 1) & 2) ? -v : v;
+    v = ((q + 1) & 2) ? -v : v;
+    return bad ? TRK_NAN : v;
 }
 
 /* sin and cos of one argument from one reduction; each equals trk_sin(x) /
  * trk_cos(x) bit for bit. */
 TRK_FN void trk_sincos(double x, double *s, double *c)
 {
-    if (x != x || trk_fabs(x) == TRK_INF) { *s = TRK_NAN; *c = TRK_NAN; return; }
+    const int bad = !(trk_fabs(x) < TRK_INF);
     int q;
-    double r = trk_reduce_pio2(x, &q);
+    double r = trk_reduce_pio2(bad ? 0.0 : x, &q);
     double sp = trk_sin_poly(r), cp = trk_cos_poly(r);
     double vs = (q & 1) ? cp : sp;
     double vc = (q & 1) ? sp : cp;
-    *s = (q & 2) ? -vs : vs;
-    *c = ((q + 1) & 2) ? -vc : vc;
+    vs = (q & 2) ? -vs : vs;
+    vc = ((q + 1) & 2) ? -vc : vc;
+    *s = bad ? TRK_NAN : vs;
+    *c = bad ? TRK_NAN : vc;
 }
 
 /* --- atan / acos ------------------------------------------------------------ */
@@ -246,23 +255,26 @@ TRK_FN double trk_atan(double x)
 {
     const double PIO2 = 0x1.921fb54442d18p+0;
     const double PIO2_LO = 0x1.1a62633145c07p-54;
-    if (x != x) return x;
     double ax = trk_fabs(x);
     const int big = ax > 1.0;
-    double a = trk_atan_small(big ? 1.0 / ax : ax);   /* one evaluation for every lane */
+    const double inv = 1.0 / ax;
+    double a = trk_atan_small(big ? inv : ax);        /* one evaluation for every lane */
     double r = big ? (PIO2 - a) + PIO2_LO : a;
-    return (x < 0.0) ? -r : r;
+    r = (x < 0.0) ? -r : r;
+    return (x != x) ? x : r;
 }
 
 TRK_FN double trk_acos(double x)
 {
     const double PI = 0x1.921fb54442d18p+1;
-    if (x != x) return x;
-    if (x > 1.0 || x < -1.0) return TRK_NAN;
-    if (x == 1.0) return 0.0;
-    if (x == -1.0) return PI;
-    double t = trk_sqrt((1.0 - x) / (1.0 + x));
-    return 2.0 * trk_atan(t);
+    const int in = x > -1.0 && x < 1.0;
+    const double xc = in ? x : 0.0;
+    double t = trk_sqrt((1.0 - xc) / (1.0 + xc));
+    double v = 2.0 * trk_atan(t);
+    double w = (x == 1.0) ? 0.0 : PI;          /* x = -1 */
+    w = (x > 1.0 || x < -1.0) ? TRK_NAN : w;
+    w = (x != x) ? x : w;
+    return in ? v : w;
 }
 
 /* --- pow ------------------------------------------------------------------ */
