@@ -122,15 +122,6 @@ TRK_HD double interpolate(int flag, double E1, double E2, double S1, double S2, 
     return S1 + ((S2 - S1) / (E2 - E1)) * (E - E1);
 }
 
-// define_dE, Cross_sections.f90:1374-1412 (new grid, both bounds present)
-TRK_HD double define_dE(int n, double E, double E0_min, double E0_max, double dE_min)
-{
-    double dE;
-    if ((E > E0_min) && (E < E0_max)) dE = (E0_max - E0_min) / (double)n;
-    else dE = E / (double)n;
-    return (dE > dE_min) ? dE : dE_min;
-}
-
 // Next_free_path_2d (MC:1874-1899) in the trk namespace, for host code (the
 // event code compiles its own copy in each of its namespaces)
 TRK_HD double nfp_2d_host(const double *Ea, const double *La, int n, double E)

@@ -14,17 +14,24 @@
 // omega node, a geometric q grid (Simpson with the left-node 1/q weight).
 // Here the work is split into four launches so that the expensive part -- the
 // q integral behind each omega node, ~10^7 of them per material -- runs one
-// per GPU thread:
-//   1. plan   (one thread per row)    walk the omega recurrence, count nodes
-//   2. nodes  (one thread per row)    write left node E_k and step dE_k
-//   3. eval   (one thread per point)  q-integral at the row start, E_k+dE_k/2, E_k+dE_k
-//   4. scan   (one thread per row)    Simpson sums in the reference's order,
+// per lane of waves that each stay inside one row:
+//   1. plan   (one wave per row)      walk the omega recurrence, count nodes
+//   2. nodes  (one wave per row)      write left node E_k and step dE_k
+//   3. eval   (one lane per point)    q-integral at the row start, E_k+dE_k/2, E_k+dE_k
+//   4. scan   (one wave per row)      Simpson sums in the reference's order,
 //                                      cumulative rows, MFP, dE/dx
 // Steps 1, 2 and 4 perform exactly the reference's floating-point operations
 // in the reference's order, and step 3 is a pure function of its inputs, so
 // the tables are bit-identical to a sequential evaluation.  The q loop is
 // VALU-bound FP64 work (a correctly rounded division per oscillator per
 // node); it has no dense contraction, so MFMA is not used.
+//
+// Measured on the MI355X (ms per build: an Al2O3-like target of seven
+// oscillators in three shells / an Al-like metal with masses from its density
+// of states / the oxide with the FP32 quadrature): eval 42 -> 9.1, 71 -> 15.6
+// and 76 -> 10 since a wave takes one row and its loop holds only what changes
+// with q (1.75e10 -> 3.4e9 wave instructions, lanes in use 49 -> 98 %), plan and
+// nodes 1.6 -> 0.9 and 2.8 -> 1.7, scan 4.6 -> 0.42 and 6.9 -> 0.76.
 #include <hip/hip_runtime.h>
 #include <algorithm>
 #include <chrono>
@@ -110,8 +117,224 @@ constexpr int kMaxQSteps = 1 << 20;
 // Nodes of one transfer-energy row (the reference's rows hold up to ~1400).
 constexpr int kMaxRowSteps = 1 << 20;
 
+// ---- the q quadrature of one point
+// Quotients of the quadrature's inner loop.  recip and quot are the steps of
+// the hardware's full division without its operand scaling and special cases:
+// the same rounded result wherever a full division would not scale, which
+// q_in_range states for a whole point before its loop starts.
+TRK_DEV double recip(double d)
+{
+    double y = __builtin_amdgcn_rcp(d);
+    y = __builtin_fma(y, __builtin_fma(-d, y, 1.0), y);
+    return __builtin_fma(y, __builtin_fma(-d, y, 1.0), y);
+}
+TRK_DEV double quot(double n, double d, double y)
+{
+    const double q = n * y;
+    return __builtin_fma(__builtin_fma(-d, q, n), y, q);
+}
+// n / c for a constant c, y the rounded 1/c.  One correction of n y is the
+// rounded quotient (Markstein's theorem) if n y lies within 1 ulp of it,
+// which |c y - 1| <= 2^-54 ensures (100 and 6); with any other c a second
+// correction follows.
+TRK_DEV double quot_const(double n, double c, double y) { return quot(n, c, y); }
+TRK_HD double quot_any(double n, double c, double y)
+{
+    double q = n * y;
+    q = __builtin_fma(__builtin_fma(-c, q, n), y, q);
+    return __builtin_fma(__builtin_fma(-c, q, n), y, q);
+}
+
+// The oscillators of a point's sum: a shell's, or the phonons.
+struct OscSpan {
+    const double *A, *E, *G;
+    int n;
+};
+
+// The effective masses of a density of states in LDS: the momenta k, and of
+// every interval the denominator (2 m*) m_e with its reciprocal.
+struct DosMass {
+    const double *k, *c, *y;
+    int nk;
+};
+constexpr int kMaxDosMass = 2048;    // 48 KB of LDS
+constexpr double kOneCv = (2.0 * 1.0) * kMe;
+
+// Every quotient of the loop stays far from the ends of the exponent range,
+// and every numerator is non-zero.
+// The bounds leave numerators in 1e-60..1e60 over denominators in
+// 1e-60..1e100, their Simpson terms in 1e-210..1e180 over momenta in
+// 1e-30..1e60, so no quotient nor reciprocal comes near 2^+-768.
+TRK_DEV bool q_in_range(const OscSpan &o, double w, double cmin, double cmax, double qmin, double qmax)
+{
+    bool ok = qmin >= 1.0e-30 && qmax <= 1.0e60 && w >= 1.0e-24 && w <= 1.0e24 && cmin >= 1.0e-60 && cmax <= 1.0e60;
+    const double top = qmax * 1.02;
+    const double smax = ((kH * kH) * top) * top;
+    ok = ok && smax <= 1.0e23 * cmin;
+    for (int i = 0; i < o.n; ++i) {
+        const double num = trk_fabs((o.A[i] * o.G[i]) * w), g2 = (o.G[i] * o.G[i]) * (w * w);
+        ok = ok && num >= 1.0e-60 && num <= 1.0e60 && g2 >= 1.0e-60 && g2 <= 1.0e60 && trk_fabs(o.E[i]) <= 1.0e23;
+    }
+    return ok;
+}
+
+// Simpson over the geometric q grid (left-node 1/q weight) of the loss
+// function with E0(q) = E + hbar^2 q^2 / c.  Bound by FP64 issue: per step
+// and oscillator two terms of 18 operations, 11 of them the quotient.  What
+// does not change along the loop (A G w, G^2 w^2, 1/c) is computed before it,
+// the step's own quotients (by 100, 6 and c) are multiplications by a rounded
+// reciprocal with correction, and both nodes of a step share one pass over
+// the oscillators.  kN oscillators (0: any number, read in the loop);
+// kDos: c follows q through the density of states; kPh: weight 1/q as a factor.
+template <int kN, bool kDos, bool kPh>
+TRK_DEV double q_simpson(const OscSpan &o, const DosMass &dm, double w, double c, double qmin, double qmax)
+{
+    constexpr int kA = kN ? kN : 1;
+    const int n = kN ? kN : o.n;
+    const double w2 = w * w;
+    double num[kA], g2[kA], E[kA];
+    if (kN) {
+#pragma unroll
+        for (int i = 0; i < kA; ++i) {
+            num[i] = (o.A[i] * o.G[i]) * w;
+            g2[i] = (o.G[i] * o.G[i]) * w2;
+            E[i] = o.E[i];
+        }
+    }
+    constexpr double y100 = 1.0 / 100.0, y6 = 1.0 / 6.0;
+    const double rootE = kDos ? trk_sqrt(kE) : 0.0;
+    double y = kDos ? 0.0 : 1.0 / c;
+    // kDos: the interval of q is the number of k entries not above it; q only
+    // grows, so it is looked for once and then followed.  One past the last
+    // entry the mass is that entry's; beyond, the free electron's.
+    int at = 0;
+    double knext = 0.0;
+    auto interval = [&](double v) {
+        while (v >= knext) {
+            ++at;
+            if (at < dm.nk) {
+                knext = dm.k[at];
+                c = dm.c[at];
+                y = dm.y[at];
+            } else if (at == dm.nk) {
+                knext = __longlong_as_double(__double_as_longlong(dm.k[dm.nk - 1]) + 1);
+                c = dm.c[dm.nk - 1];
+                y = dm.y[dm.nk - 1];
+            } else {
+                knext = __builtin_inf();
+                c = kOneCv;
+                y = recip(kOneCv);
+            }
+        }
+    };
+    if (kDos) {
+        const double v = qmin * rootE;
+        int lo = -1, hi = dm.nk;      // k[lo] <= v < k[hi]
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) >> 1;
+            if (dm.k[mid] <= v) lo = mid;
+            else hi = mid;
+        }
+        at = hi - 1;
+        knext = -__builtin_inf();     // the first look sets c and y
+        interval(v);
+    }
+    double dLs = 0.0, hq = qmin, dLs0 = 0.0;
+    for (int g = 0; hq < qmax && g < kMaxQSteps; ++g) {
+        const double dq = quot_const(hq, 100.0, y100);
+        const double a = hq + dq * 0.5;
+        const double b = hq + dq;
+        const double ha = ((kH * kH) * a) * a, hb = ((kH * kH) * b) * b;
+        double sa, sb;
+        if (kDos) {
+            interval(a * rootE);
+            sa = quot(ha, c, y);
+            interval(b * rootE);
+            sb = quot(hb, c, y);
+        } else {
+            sa = quot_any(ha, c, y);
+            sb = quot_any(hb, c, y);
+        }
+        double Fa = 0.0, Fb = 0.0;
+#pragma unroll
+        for (int i = 0; i < n; ++i) {
+            const double nu = kN ? num[kN ? i : 0] : (o.A[i] * o.G[i]) * w;
+            const double gg = kN ? g2[kN ? i : 0] : (o.G[i] * o.G[i]) * w2;
+            const double Ei = kN ? E[kN ? i : 0] : o.E[i];
+            const double Ea = Ei + sa, Eb = Ei + sb;
+            const double xa = w2 - Ea * Ea, xb = w2 - Eb * Eb;
+            const double da = xa * xa + gg, db = xb * xb + gg;
+            Fa = Fa + quot(nu, da, recip(da));
+            Fb = Fb + quot(nu, db, recip(db));
+        }
+        const double t = quot_const(dq, 6.0, y6) * ((dLs0 + 4.0 * Fa) + Fb);
+        const double yq = recip(hq);
+        dLs = dLs + (kPh ? t * quot(1.0, hq, yq) : quot(t, hq, yq));
+        dLs0 = Fb;
+        hq = b;
+    }
+    return dLs;
+}
+
+template <bool kDos, bool kPh>
+TRK_DEV double q_simpson_n(const OscSpan &o, const DosMass &dm, double w, double c, double qmin, double qmax)
+{
+    switch (o.n) {
+    case 1: return q_simpson<1, kDos, kPh>(o, dm, w, c, qmin, qmax);
+    case 2: return q_simpson<2, kDos, kPh>(o, dm, w, c, qmin, qmax);
+    case 3: return q_simpson<3, kDos, kPh>(o, dm, w, c, qmin, qmax);
+    case 4: return q_simpson<4, kDos, kPh>(o, dm, w, c, qmin, qmax);
+    case 5: return q_simpson<5, kDos, kPh>(o, dm, w, c, qmin, qmax);
+    default: return q_simpson<0, kDos, kPh>(o, dm, w, c, qmin, qmax);
+    }
+}
+
+// The q integral of one point: the form above for the free-electron
+// dispersion, else (plasmon-pole and Ritchie dispersions, densities of states
+// whose k do not increase, values outside q_in_range in any lane) the loss
+// function as it is written.  shell < 0: the phonons.  All lanes of a wave
+// come here with the same shell.
+TRK_DEV double q_integral(const MatDev &m, const DosMass &dm, int shell, double w, double qmin, double qmax)
+{
+    const bool ph = shell < 0;
+    OscSpan o;
+    if (ph) o = OscSpan{m.phA, m.phE0, m.phG, m.n_ph};
+    else {
+        const int o0 = m.osc_off[shell];
+        o = OscSpan{m.oA + o0, m.oE0 + o0, m.oG + o0, m.osc_off[shell + 1] - o0};
+    }
+    const bool dos = !ph && m.use_k;
+    if ((ph || (m.kind_of_DR != 2 && m.kind_of_DR != 3)) && (!dos || dm.nk > 0)) {
+        double c;
+        if (ph) c = 2.0 * m.Mtarget;
+        else c = (2.0 * ((m.El_eff_mass > 0.0) ? m.El_eff_mass : 1.0)) * kMe;
+        // the masses of a usable density of states lie in 1e-6..1e6
+        const bool ok = dos ? q_in_range(o, w, 1.0e-6 * kOneCv, 1.0e6 * kOneCv, qmin, qmax) : q_in_range(o, w, c, c, qmin, qmax);
+        if (!__any(!ok && qmin < qmax)) {
+            if (ph) return q_simpson_n<false, true>(o, dm, w, c, qmin, qmax);
+            if (dos) return q_simpson_n<true, false>(o, dm, w, c, qmin, qmax);
+            return q_simpson_n<false, false>(o, dm, w, c, qmin, qmax);
+        }
+    }
+    double dLs = 0.0, hq = qmin, dLs0 = 0.0;
+    for (int g = 0; (ph ? trk_fabs(hq) < trk_fabs(qmax) : hq < qmax) && g < kMaxQSteps; ++g) {
+        double dq = hq / 100.0;
+        double a = hq + dq / 2.0;
+        double b = hq + dq;
+        double temp1 = 0.0, dL = 0.0;
+        for (int i = 0; i < o.n; ++i) temp1 = temp1 + loss(m, ph ? 2 : 0, o.A[i], o.E[i], o.G[i], w, a);
+        for (int i = 0; i < o.n; ++i) dL = dL + loss(m, ph ? 2 : 0, o.A[i], o.E[i], o.G[i], w, b);
+        const double t = (dq / 6.0) * ((dLs0 + 4.0 * temp1) + dL);
+        if (ph) dLs = dLs + t * (1.0 / hq);
+        else dLs = dLs + t / hq;
+        dLs0 = dL;
+        hq = hq + dq;
+    }
+    return dLs;
+}
+
 // Diff_cross_section, Cross_sections.f90:2217-2282
-TRK_DEV double diff_cs(const MatDev &m, int shell, double Ee, double dE, double Mass)
+TRK_DEV double diff_cs(const MatDev &m, const DosMass &dm, int shell, double Ee, double dE, double Mass)
 {
     double qmin, qmax;
     double pre = trk_sqrt((2.0 * Mass) * kMe) / kH;
@@ -122,23 +345,13 @@ TRK_DEV double diff_cs(const MatDev &m, int shell, double Ee, double dE, double 
         qmin = pre * (trk_sqrt(Ee) - trk_sqrt(Ee - dE));
         qmax = pre * (trk_sqrt(Ee) + trk_sqrt(Ee - dE));
     }
-    double dLs = 0.0, hq = qmin, dLs0 = 0.0;
-    for (int g = 0; hq < qmax && g < kMaxQSteps; ++g) {
-        double dq = hq / 100.0;
-        double a = hq + dq / 2.0;
-        double temp1 = imewq(m, dE, a, shell, 0);
-        double b = hq + dq;
-        double dL = imewq(m, dE, b, shell, 0);
-        dLs = dLs + ((dq / 6.0) * ((dLs0 + 4.0 * temp1) + dL)) / hq;
-        dLs0 = dL;
-        hq = hq + dq;
-    }
+    const double dLs = q_integral(m, dm, shell, dE, qmin, qmax);
     double T_fact = (m.temp > 0.0) ? 1.0 / (1.0 - trk_exp(-((dE / m.temp) * kKb))) : 1.0;
     return ((1.0 / ((kPi * kA0) * Ee)) * dLs) * T_fact;
 }
 
 // Diff_cross_section_phonon, Cross_sections.f90:3142-3300 (screening 1)
-TRK_DEV double diff_cs_phonon(const MatDev &m, double Ee, double dE, double Mass)
+TRK_DEV double diff_cs_phonon(const MatDev &m, const DosMass &dm, double Ee, double dE, double Mass)
 {
     const double eps = 1.0e-12;
     double qmin, qmax;
@@ -147,43 +360,21 @@ TRK_DEV double diff_cs_phonon(const MatDev &m, double Ee, double dE, double Mass
     else if (dE > (Ee - eps)) qmin = pre * trk_sqrt(Ee);
     else qmin = pre * (trk_sqrt(Ee) - trk_sqrt(trk_fabs(Ee - dE)));
     qmax = ((1.0 * trk_sqrt((2.0 * Mass) * kMe)) / kH) * (trk_sqrt(Ee) + trk_sqrt(trk_fabs(Ee - dE)));
-    double dLs = 0.0, hq = qmin, dLs0 = 0.0;
-    for (int g = 0; trk_fabs(hq) < trk_fabs(qmax) && g < kMaxQSteps; ++g) {
-        double dq = hq / 100.0;
-        double a = hq + dq / 2.0;
-        double temp1 = 0.0, dL = 0.0;
-        for (int i = 0; i < m.n_ph; ++i) temp1 = temp1 + loss(m, 2, m.phA[i], m.phE0[i], m.phG[i], dE, a);
-        double b = hq + dq;
-        for (int i = 0; i < m.n_ph; ++i) dL = dL + loss(m, 2, m.phA[i], m.phE0[i], m.phG[i], dE, b);
-        double Pot = 1.0 / hq;
-        dLs = dLs + ((dq / 6.0) * ((dLs0 + 4.0 * temp1) + dL)) * Pot;
-        dLs0 = dL;
-        hq = hq + dq;
-    }
+    const double dLs = q_integral(m, dm, -1, dE, qmin, qmax);
     if (m.temp > 1.0e-6)
         return ((1.0 / ((kPi * kA0) * Ee)) * dLs) / (1.0 - trk_exp(-((dE / m.temp) * kKb)));
     return (1.0 / ((kPi * kA0) * Ee)) * dLs;
 }
 
 // SHI_Diff_cross_section, Cross_sections.f90:2683-2744
-TRK_DEV double shi_diff_cs(const MatDev &m, int shell, double Ee, double MSHI, double Emax, double hw)
+TRK_DEV double shi_diff_cs(const MatDev &m, const DosMass &dm, int shell, double Ee, double MSHI, double Emax, double hw)
 {
     double qmin, qmax;
     if (Ee > 0.0) qmin = (hw / kH) / trk_sqrt((2.0 * Ee) / MSHI);
     else qmin = 0.0;
     if (Emax > 0.0) qmax = (trk_sqrt(2.0 * kMe) / kH) * trk_sqrt(Emax);
     else return 0.0;
-    double dLs = 0.0, hq = qmin, dLs0 = 0.0;
-    for (int g = 0; hq < qmax && g < kMaxQSteps; ++g) {
-        double dq = hq / 100.0;
-        double a = hq + dq / 2.0;
-        double temp1 = imewq(m, hw, a, shell, 0);
-        double b = hq + dq;
-        double dL = imewq(m, hw, b, shell, 0);
-        dLs = dLs + ((dq / 6.0) * ((dLs0 + 4.0 * temp1) + dL)) / hq;
-        dLs0 = dL;
-        hq = hq + dq;
-    }
+    const double dLs = q_integral(m, dm, shell, hw, qmin, qmax);
     double T_fact = (m.temp > 0.0) ? 1.0 / (1.0 - trk_exp(-((hw / m.temp) * kKb))) : 1.0;
     return dLs * T_fact;
 }
@@ -289,6 +480,78 @@ TRK_DEV float imewq32(const MatDev &m, int shell, float w, float q2, float inv_m
     return ImE;
 }
 
+// n / d in FP32: the steps of the hardware's full division without its
+// scaling and special cases, the same rounded result inside in_range32.
+TRK_DEV float quot32(float n, float d)
+{
+    float y = __builtin_amdgcn_rcpf(d);
+    y = __builtin_fmaf(__builtin_fmaf(-d, y, 1.0f), y, y);
+    float q = n * y;
+    q = __builtin_fmaf(__builtin_fmaf(-d, q, n), y, q);
+    return __builtin_fmaf(__builtin_fmaf(-d, q, n), y, q);
+}
+
+// Numerators in 1e-6..1e10 over denominators in 1e-12..1e30: quotients of
+// 1e-36..1e22, where no operand is scaled.
+TRK_DEV bool in_range32(const OscSpan &o, float w, double qhi, float inv_mstar)
+{
+    const float smax = ((float)qhi * (float)qhi) * 1.01f * inv_mstar;
+    bool ok = w >= 1.0e-7f && w <= 1.0e7f && smax >= 0.0f && smax <= 1.0e7f;
+    for (int i = 0; i < o.n; ++i) {
+        const float E = (float)o.E[i], G = (float)o.G[i], A = (float)o.A[i];
+        const float num = fabsf(A * G * w), g2 = G * G * (w * w);
+        ok = ok && num >= 1.0e-6f && num <= 1.0e10f && g2 >= 1.0e-12f && g2 <= 1.0e28f && E >= 0.0f && E <= 1.0e7f;
+    }
+    return ok;
+}
+
+// The Simpson sum over ln q with the free-electron dispersion and kN
+// oscillators (0: any number).  Bound by FP32 issue, one quotient per
+// oscillator and node; the numerators and widths are converted and
+// multiplied once per point.
+template <int kN>
+TRK_DEV double q32_simpson(const OscSpan &o, float w, float u0, float h, float inv_mstar)
+{
+    constexpr int kA = kN ? kN : 1;
+    const int n = kN ? kN : o.n;
+    const float w2 = w * w;
+    float num[kA], g2[kA], E[kA];
+    if (kN) {
+#pragma unroll
+        for (int i = 0; i < kA; ++i) {
+            const float G = (float)o.G[i], A = (float)o.A[i];
+            num[i] = A * G * w;
+            g2[i] = G * G * w2;
+            E[i] = (float)o.E[i];
+        }
+    }
+    auto term = [&](int k) {
+        const float q = __expf(u0 + h * (float)k);
+        const float sqq = (q * q) * inv_mstar;
+        float f = 0.0f;
+#pragma unroll
+        for (int i = 0; i < n; ++i) {
+            const float G = kN ? 0.0f : (float)o.G[i];
+            const float nu = kN ? num[kN ? i : 0] : (float)o.A[i] * G * w;
+            const float gg = kN ? g2[kN ? i : 0] : G * G * w2;
+            const float E0 = (kN ? E[kN ? i : 0] : (float)o.E[i]) + sqq;
+            const float d = w2 - E0 * E0;
+            f = f + quot32(nu, d * d + gg);
+        }
+        return f;
+    };
+    Kahan32 S;
+    S.add(1.0f * term(0));
+    for (int k = 1; k + 1 < kQ32Q; k += 2) {
+        const float f1 = term(k), f2 = term(k + 1);
+        S.add(4.0f * f1);
+        S.add(2.0f * f2);
+    }
+    S.add(4.0f * term(kQ32Q - 1));
+    S.add(1.0f * term(kQ32Q));
+    return S.value();
+}
+
 // One point of a row: the q integral of Diff_cross_section (CS:2217-2282) or
 // SHI_Diff_cross_section (CS:2683-2744) at transfer energy x, in FP32.
 TRK_DEV double eval32(const MatDev &m, const RowJob &j, double x)
@@ -314,129 +577,209 @@ TRK_DEV double eval32(const MatDev &m, const RowJob &j, double x)
     const float c_vf = (float)(((m.v_f * m.v_f) * (2.0 * kMe)) / 3.0);
     const float u0 = (float)trk_log(qlo), h = (float)((trk_log(qhi) - trk_log(qlo)) / (double)kQ32Q);
     const float w = (float)x;
-    Kahan32 S;
-    for (int k = 0; k <= kQ32Q; ++k) {
-        const float q = __expf(u0 + h * (float)k);
-        const float f = imewq32(m, j.shell, w, q * q, inv_mstar, c_vf);
-        const float wk = (k == 0 || k == kQ32Q) ? 1.0f : ((k & 1) ? 4.0f : 2.0f);
-        S.add(wk * f);
+    const int s0 = m.osc_off[j.shell];
+    const OscSpan o{m.oA + s0, m.oE0 + s0, m.oG + s0, m.osc_off[j.shell + 1] - s0};
+    double S;
+    if (m.kind_of_DR != 2 && m.kind_of_DR != 3 && !__any(!in_range32(o, w, qhi, inv_mstar))) {
+        switch (o.n) {
+        case 1: S = q32_simpson<1>(o, w, u0, h, inv_mstar); break;
+        case 2: S = q32_simpson<2>(o, w, u0, h, inv_mstar); break;
+        case 3: S = q32_simpson<3>(o, w, u0, h, inv_mstar); break;
+        case 4: S = q32_simpson<4>(o, w, u0, h, inv_mstar); break;
+        case 5: S = q32_simpson<5>(o, w, u0, h, inv_mstar); break;
+        default: S = q32_simpson<0>(o, w, u0, h, inv_mstar); break;
+        }
+    } else {
+        Kahan32 K;
+        for (int k = 0; k <= kQ32Q; ++k) {
+            const float q = __expf(u0 + h * (float)k);
+            const float f = imewq32(m, j.shell, w, q * q, inv_mstar, c_vf);
+            const float wk = (k == 0 || k == kQ32Q) ? 1.0f : ((k & 1) ? 4.0f : 2.0f);
+            K.add(wk * f);
+        }
+        S = K.value();
     }
-    return (double)((float)pref * ((h / 3.0f) * (float)S.value()));
+    return (double)((float)pref * ((h / 3.0f) * (float)S));
 }
 
+// define_dE (CS:1374-1412) along a row, the nodes E_k+1 = E_k + dE(E_k).  One
+// chain of dependent operations per row, so a wave walks it for all its
+// lanes, 64 steps without a branch (lane t keeps node t), and the quotient by
+// n is a multiplication by its rounded reciprocal with one correction
+// (quot_const; a full division where n or the range do not allow it).
+struct RowWalk {
+    double n, y, lo, hi, inner, dE_min;
+    bool quick;
+    TRK_DEV explicit RowWalk(const RowJob &j)
+        : n((double)j.n), y(1.0 / (double)j.n), lo(j.E_low), hi(j.E_high), inner((j.E_high - j.E_low) / (double)j.n),
+          dE_min(j.dE_min)
+    {
+        quick = j.Estart >= 1.0e-200 && j.E_low >= 1.0e-200 && j.Emax <= 1.0e200 &&
+                trk_fabs(__builtin_fma(n, y, -1.0)) <= 0x1.0p-54;
+    }
+    template <bool kQuick>
+    TRK_DEV double step(double E) const
+    {
+        const double q = kQuick ? quot_const(E, n, y) : E / n;
+        const double dE = ((E > lo) & (E < hi)) ? inner : q;
+        return (dE > dE_min) ? dE : dE_min;
+    }
+    template <bool kQuick>
+    TRK_DEV void walk(double &E, double &node, double &width) const
+    {
+        const int lane = threadIdx.x & 63;
+#pragma unroll 8
+        for (int t = 0; t < 64; ++t) {
+            const double dE = step<kQuick>(E);
+            if (lane == t) {
+                node = E;
+                width = dE;
+            }
+            E = E + dE;
+        }
+    }
+    // the next 64 nodes from E on, and their steps; E moves behind them
+    TRK_DEV void next(double &E, double &node, double &width) const
+    {
+        if (quick) walk<true>(E, node, width);
+        else walk<false>(E, node, width);
+    }
+    // nodes from E on up to Emax
+    TRK_DEV int count(double E, double Emax) const
+    {
+        for (int c = 0; c < kMaxRowSteps; c += 64) {
+            double node = 0.0, width = 0.0;
+            next(E, node, width);
+            const unsigned long long in = __ballot(node <= Emax);
+            if (~in) return c + __builtin_ctzll(~in);
+        }
+        return kMaxRowSteps;
+    }
+};
+
+// One wave per row.
 __global__ void k_row_plan(const RowJob *__restrict__ jobs, int nrows, int *__restrict__ cnt, int *__restrict__ len)
 {
-    int r = blockIdx.x * blockDim.x + threadIdx.x;
+    const int r = blockIdx.x * (blockDim.x / 64) + __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64);
     if (r >= nrows) return;
-    RowJob j = jobs[r];
-    int c = 0;
-    double E = j.Estart;
+    const RowJob j = jobs[r];
+    int c = 0, L = 0;
     if (j.q32) {
         // the fixed geometric intervals of the FP32 quadrature (none when
         // the range is empty); rows hold at least 10 entries, as the
         // reference's allocation does
         c = (j.Emax > j.Estart && j.Estart > 0.0) ? kQ32W : 0;
-        cnt[r] = c;
-        len[r] = j.with_row ? ((j.type == ROW_SHI_DIFF) ? c : (c > 10 ? c : 10)) : 0;
-        return;
-    }
-    if (j.type == ROW_PHONON) {
-        while (trk_fabs(E) <= trk_fabs(j.Emax) && c < kMaxRowSteps) {
-            c++;
-            E = E + 1.0 * define_dE(j.n, E, j.E_low, j.E_high, j.dE_min);
-        }
+        if (j.with_row) L = (j.type == ROW_SHI_DIFF) ? c : (c > 10 ? c : 10);
     } else {
-        while (E <= j.Emax && c < kMaxRowSteps) {
-            c++;
-            E = E + define_dE(j.n, E, j.E_low, j.E_high, j.dE_min);
-        }
-    }
-    if (c >= kMaxRowSteps) { cnt[r] = -1; len[r] = 0; return; }
-    int L = 0;
-    if (j.with_row) {
-        if (j.type == ROW_SHI_DIFF) {
-            L = c;
-        } else {
-            // allocation count of get_diff_CS_grid_size (CS:1278-1343): from E_low
-            int nref = 0;
-            double Er = j.E_low;
-            while (Er <= j.Emax && nref < kMaxRowSteps) {
-                nref++;
-                Er = Er + define_dE(j.n, Er, j.E_low, j.E_high, j.dE_min);
+        const RowWalk w(j);
+        // phonon rows compare the magnitudes; they start at a positive energy
+        c = (j.type == ROW_PHONON) ? w.count(j.Estart, trk_fabs(j.Emax)) : w.count(j.Estart, j.Emax);
+        if (c >= kMaxRowSteps) {
+            c = -1;
+        } else if (j.with_row) {
+            if (j.type == ROW_SHI_DIFF) {
+                L = c;
+            } else {
+                // allocation count of get_diff_CS_grid_size (CS:1278-1343): from E_low
+                const int nref = w.count(j.E_low, j.Emax);
+                L = c;
+                if (nref > L) L = nref;
+                if (L < 10) L = 10;
             }
-            L = c;
-            if (nref > L) L = nref;
-            if (L < 10) L = 10;
         }
     }
-    cnt[r] = c;
-    len[r] = L;
+    if ((threadIdx.x & 63) == 0) {
+        cnt[r] = c;
+        len[r] = L;
+    }
 }
+
+// Points of a row: its start, then the midpoint and the right node of every
+// step.  A wave of k_eval takes kPointsWave points of one row.
+constexpr int kPointsWave = 64;
+constexpr int kEvalBlock = 256;
+TRK_HD int64_t row_chunks(int64_t steps) { return (2 * steps + 1 + kPointsWave - 1) / kPointsWave; }
 
 __global__ void k_row_nodes(const RowJob *__restrict__ jobs, int nrows, const int64_t *__restrict__ step_off,
-                            double *__restrict__ Ek, double *__restrict__ dEk, int *__restrict__ step_row)
+                            const int64_t *__restrict__ chunk_off, double *__restrict__ Ek, double *__restrict__ dEk,
+                            int *__restrict__ chunk_row)
 {
-    int r = blockIdx.x * blockDim.x + threadIdx.x;
+    const int lane = threadIdx.x & 63;
+    const int r = blockIdx.x * (blockDim.x / 64) + __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64);
     if (r >= nrows) return;
-    RowJob j = jobs[r];
-    int64_t o = step_off[r];
-    int64_t o1 = step_off[r + 1];
-    double E = j.Estart;
+    const RowJob j = jobs[r];
+    const int64_t o = step_off[r], n = step_off[r + 1] - o;
+    for (int64_t c = chunk_off[r] + lane; c < chunk_off[r + 1]; c += 64) chunk_row[c] = r;
     if (j.q32) {
         const double lr = trk_log(j.Emax / j.Estart) / (double)kQ32W;
-        for (int64_t k = o; k < o1; ++k) {
-            const int64_t i = k - o;
+        for (int64_t i = lane; i < n; i += 64) {
             const double a = j.Estart * trk_exp(lr * (double)i);
-            const double b = (i + 1 == o1 - o) ? j.Emax : j.Estart * trk_exp(lr * (double)(i + 1));
-            Ek[k] = a;
-            dEk[k] = b - a;
-            step_row[k] = r;
+            const double b = (i + 1 == n) ? j.Emax : j.Estart * trk_exp(lr * (double)(i + 1));
+            Ek[o + i] = a;
+            dEk[o + i] = b - a;
         }
         return;
     }
-    for (int64_t k = o; k < o1; ++k) {
-        double dE = define_dE(j.n, E, j.E_low, j.E_high, j.dE_min);
-        if (j.type == ROW_PHONON) dE = 1.0 * dE;
-        Ek[k] = E;
-        dEk[k] = dE;
-        step_row[k] = r;
-        E = E + dE;
+    const RowWalk w(j);
+    double E = j.Estart;
+    for (int64_t i = 0; i < n; i += 64) {
+        double node = 0.0, width = 0.0;
+        w.next(E, node, width);
+        if (i + lane < n) {
+            Ek[o + i + lane] = node;
+            dEk[o + i + lane] = width;
+        }
     }
 }
 
-TRK_DEV double eval_point(const MatDev &m, const RowJob &j, double x)
+TRK_DEV double eval_point(const MatDev &m, const DosMass &dm, const RowJob &j, double x)
 {
     if (j.q32) return eval32(m, j, x);
     switch (j.type) {
-    case ROW_INEL: return diff_cs(m, j.shell, j.Ele, x, j.Mass);
-    case ROW_PHONON: return diff_cs_phonon(m, j.Ele, x, j.Mass);
+    case ROW_INEL: return diff_cs(m, dm, j.shell, j.Ele, x, j.Mass);
+    case ROW_PHONON: return diff_cs_phonon(m, dm, j.Ele, x, j.Mass);
     default:
         if (j.bk) return shi_diff_cs_bk(m, j.shell, j.Ele, j.MSHI, j.Emax, x, j.Zp, j.Zeff);
-        return shi_diff_cs(m, j.shell, j.Ele, j.MSHI, j.Emax, x);
+        return shi_diff_cs(m, dm, j.shell, j.Ele, j.MSHI, j.Emax, x);
     }
 }
 
-// Points [0, nrows) are the row starts; points nrows + 2k (+1) are the
-// midpoint and right node of step k.
-__global__ void k_eval(MatDev m, const RowJob *__restrict__ jobs, int nrows, int64_t nsteps,
-                       const double *__restrict__ Ek, const double *__restrict__ dEk,
-                       const int *__restrict__ step_row, double *__restrict__ f0,
-                       double *__restrict__ fa, double *__restrict__ fb)
+// One q integral per lane, a wave's points all of one row: the row's job, its
+// shell's oscillators and the number of them are then scalars, and
+// neighbouring lanes take nearly the same number of q steps.  A row ends
+// its last wave short (half a wave of some hundred points).  dos_n: entries of
+// the density of states to stage for the masses (0: none).
+__global__ void __launch_bounds__(kEvalBlock, 6)
+k_eval(MatDev m, const RowJob *__restrict__ jobs, const int *__restrict__ chunk_row,
+       const int64_t *__restrict__ chunk_off, const int64_t *__restrict__ step_off, int64_t nchunks,
+       const double *__restrict__ Ek, const double *__restrict__ dEk, double *__restrict__ f0,
+       double *__restrict__ fa, double *__restrict__ fb, int dos_n)
 {
-    int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    int64_t total = (int64_t)nrows + 2 * nsteps;
-    if (p >= total) return;
-    if (p < nrows) {
-        RowJob j = jobs[p];
-        f0[p] = eval_point(m, j, j.Estart);
-        return;
+    extern __shared__ double lds[];
+    for (int i = threadIdx.x; i < dos_n; i += kEvalBlock) {
+        const double c = (2.0 * m.Effm[i]) * kMe;
+        lds[i] = m.k[i];
+        lds[dos_n + i] = c;
+        lds[2 * dos_n + i] = recip(c);
     }
-    int64_t q = p - nrows;
-    int64_t k = q >> 1;
-    RowJob j = jobs[step_row[k]];
-    double E = Ek[k], dE = dEk[k];
-    if ((q & 1) == 0) fa[k] = eval_point(m, j, E + dE / 2.0);
-    else fb[k] = eval_point(m, j, E + dE);
+    __syncthreads();
+    const int lane = threadIdx.x & 63;
+    const int64_t c0 = (int64_t)blockIdx.x * (kEvalBlock / kPointsWave) +
+                       __builtin_amdgcn_readfirstlane((int)threadIdx.x / kPointsWave);
+    if (c0 >= nchunks) return;
+    const int r = __builtin_amdgcn_readfirstlane(chunk_row[c0]);
+    const RowJob j = jobs[r];
+    const int64_t o = step_off[r];
+    const int64_t p = (c0 - chunk_off[r]) * kPointsWave + lane;
+    if (p > 2 * (step_off[r + 1] - o)) return;
+    const DosMass dm{lds, lds + dos_n, lds + 2 * dos_n, dos_n};
+    const int64_t k = o + ((p - 1) >> 1);
+    double x = j.Estart;
+    if (p > 0) x = Ek[k] + ((p & 1) ? dEk[k] / 2.0 : dEk[k]);
+    const double f = eval_point(m, dm, j, x);
+    if (p == 0) f0[r] = f;
+    else if (p & 1) fa[k] = f;
+    else fb[k] = f;
 }
 
 // inv[k] = 1/L[k] for one row of the ion's transfer table; *nonmono is set
@@ -461,18 +804,21 @@ __global__ void k_log(const double *__restrict__ x, int64_t n, double *__restric
 
 // mono[slot] = 1 if lam of the row never increases (and holds no NaN): the
 // row search can then count entries instead of bisecting
+// One wave per row, 64 entries at a time.
 __global__ void k_row_mono(const int64_t *__restrict__ off, int64_t nslots, const double *__restrict__ lam,
                            unsigned char *__restrict__ mono)
 {
-    int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t k = (int64_t)blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64;
     if (k >= nslots) return;
     const int64_t a = off[k], b = off[k + 1];
-    unsigned char m = 1;
-    for (int64_t i = a; i < b; ++i) {
-        if (!(lam[i] == lam[i])) m = 0;
-        if (i + 1 < b && !(lam[i] >= lam[i + 1])) m = 0;
+    bool bad = false;
+    for (int64_t i = a + (threadIdx.x & 63); i < b; i += 64) {
+        const double v = lam[i];
+        if (!(v == v)) bad = true;
+        if (i + 1 < b && !(v >= lam[i + 1])) bad = true;
     }
-    mono[k] = m;
+    const bool any = __any(bad);
+    if ((threadIdx.x & 63) == 0) mono[k] = any ? 0 : 1;
 }
 
 struct RowOut {
@@ -482,6 +828,18 @@ struct RowOut {
     const int64_t *row_off;  // [nsh*n+1]
 };
 
+TRK_DEV double lane_value(double v, int lane)
+{
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                            __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+
+// One wave per row, 64 steps at a time: the lanes load the steps' values
+// coalesced, compute their Simpson terms, and the wave adds them one after the
+// other in the row's order (each sum is a chain of rounded additions, so
+// its order is the result); every lane keeps its own partial sum and
+// writes its entry of the row.  A thread per row waited for memory at every
+// step instead.
 __global__ void k_row_scan(const RowJob *__restrict__ jobs, int nrows, const int64_t *__restrict__ step_off,
                            const double *__restrict__ Ek, const double *__restrict__ dEk,
                            const double *__restrict__ f0, const double *__restrict__ fa,
@@ -489,11 +847,11 @@ __global__ void k_row_scan(const RowJob *__restrict__ jobs, int nrows, const int
                            double *__restrict__ dE_rows, double *__restrict__ dL_rows,
                            const int64_t *__restrict__ drow_off)
 {
-    int r = blockIdx.x * blockDim.x + threadIdx.x;
+    const int lane = threadIdx.x & 63;
+    const int r = blockIdx.x * (blockDim.x / 64) + __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64);
     if (r >= nrows) return;
-    RowJob j = jobs[r];
-    int64_t o = step_off[r], o1 = step_off[r + 1];
-    double Ltot1 = 0.0, Ltot0 = f0[r], ddEdx = 0.0;
+    const RowJob j = jobs[r];
+    const int64_t o = step_off[r], o1 = step_off[r + 1];
     const RowOut &out = outs[j.kind];
     double *hw = nullptr, *cum = nullptr;
     int64_t rlen = 0;
@@ -508,61 +866,76 @@ __global__ void k_row_scan(const RowJob *__restrict__ jobs, int nrows, const int
         dEr = dE_rows + drow_off[j.shell];
         dLr = dL_rows + drow_off[j.shell];
     }
-    int64_t i = 0;
-    if (j.q32) {
-        // FP32 Simpson over the transfer-energy intervals with compensated
-        // sums; the cumulative values leave in FP64 for the normalisation
-        Kahan32 S, D;
-        float L0 = (float)Ltot0;
-        for (int64_t k = o; k < o1; ++k, ++i) {
-            const double E = Ek[k], dE = dEk[k];
-            const float La = (float)fa[k], Lb = (float)fb[k];
+    const double Z2M = (j.Zeff * j.Zeff) * j.Mass;
+    // an entry of the row: the transfer energy at the step's end and the mean
+    // free path of the sum up to it
+    auto entry = [&](int64_t i, double e, double sum) {
+        hw[i] = e;
+        if (j.type == ROW_INEL) sum = (sum < 1.0e-15) ? 1.0e15 : 1.0 / (j.Mass * sum);
+        else if (j.type == ROW_PHONON) sum = (sum < 1.0e-15) ? 1.0e20 : 1.0 / (Z2M * sum);
+        cum[i] = sum;
+    };
+    const bool weighted = (j.type == ROW_SHI && !j.bk) || j.type == ROW_SHI_DIFF;
+    double Ltot1 = 0.0, ddEdx = 0.0, prev = f0[r];
+    Kahan32 S, D;
+    for (int64_t base = o; base < o1; base += 64) {
+        const int m = (int)((o1 - base < 64) ? o1 - base : 64);
+        const int64_t k = base + ((lane < m) ? lane : m - 1);
+        const double E = Ek[k], dE = dEk[k];
+        const double temp1 = fa[k], dL = fb[k];
+        const double left = __shfl_up(dL, 1);
+        const double Ltot0 = lane ? left : prev;
+        prev = lane_value(dL, m - 1);
+        double part;
+        if (j.q32) {
+            // FP32 Simpson over the transfer-energy intervals with compensated
+            // sums; the cumulative values leave in FP64 for the normalisation
+            const float L0 = (float)Ltot0, La = (float)temp1, Lb = (float)dL;
             const float t2 = (float)(dE / 6.0) * ((L0 + 4.0f * La) + Lb);
-            S.add(t2);
             // stopping power: Simpson on w * dsigma/dw over the interval
             const float a = (float)(E + dE / 2.0), b = (float)(E + dE);
-            D.add((float)(dE / 6.0) * (((float)E * L0 + (a * 4.0f) * La) + b * Lb));
-            L0 = Lb;
-            if (hw) {
-                hw[i] = E + dE;
-                cum[i] = S.value();
+            const float td = (float)(dE / 6.0) * (((float)E * L0 + (a * 4.0f) * La) + b * Lb);
+            Kahan32 mine;
+            for (int t = 0; t < m; ++t) {
+                S.add(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(t2), t)));
+                D.add(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(td), t)));
+                if (lane == t) mine = S;
             }
+            part = mine.value();
+        } else {
+            double temp2, dd;
+            if (j.type == ROW_PHONON) temp2 = (trk_fabs(dE) / 6.0) * ((Ltot0 + 4.0 * temp1) + dL);
+            else temp2 = (dE / 6.0) * ((Ltot0 + 4.0 * temp1) + dL);
+            if (weighted) {
+                double a = E + dE / 2.0;
+                double b = E + dE;
+                dd = (dE / 6.0) * (((E * Ltot0) + ((a * 4.0) * temp1)) + (b * dL));
+            } else {
+                dd = E * temp2;
+            }
+            part = 0.0;
+            for (int t = 0; t < m; ++t) {
+                Ltot1 = Ltot1 + lane_value(temp2, t);
+                ddEdx = ddEdx + lane_value(dd, t);
+                if (lane == t) part = Ltot1;
+            }
+        }
+        if (lane < m) {
+            const int64_t i = base - o + lane;
+            if (hw) entry(i, E + dE, part);
             if (dEr) {
                 dEr[i] = E;
-                dLr[i] = (((kPi * kA0) * j.Ele) * kMe) / (((j.MSHI * j.Zeff) * j.Zeff) * S.value());
+                dLr[i] = (((kPi * kA0) * j.Ele) * kMe) / (((j.MSHI * j.Zeff) * j.Zeff) * part);
             }
         }
+    }
+    if (j.q32) {
         Ltot1 = S.value();
         ddEdx = D.value();
-        o1 = o;      // the FP64 loop below has nothing left to do
     }
-    for (int64_t k = o; k < o1; ++k, ++i) {
-        double E = Ek[k], dE = dEk[k];
-        double temp1 = fa[k], dL = fb[k];
-        double temp2;
-        if (j.type == ROW_PHONON) temp2 = (trk_fabs(dE) / 6.0) * ((Ltot0 + 4.0 * temp1) + dL);
-        else temp2 = (dE / 6.0) * ((Ltot0 + 4.0 * temp1) + dL);
-        Ltot1 = Ltot1 + temp2;
-        if ((j.type == ROW_SHI && !j.bk) || j.type == ROW_SHI_DIFF) {
-            double a = E + dE / 2.0;
-            double b = E + dE;
-            ddEdx = ddEdx + (dE / 6.0) * (((E * Ltot0) + ((a * 4.0) * temp1)) + (b * dL));
-        } else {
-            ddEdx = ddEdx + E * temp2;
-        }
-        Ltot0 = dL;
-        if (hw) {
-            hw[i] = E + dE;
-            cum[i] = Ltot1;
-        }
-        if (dEr) {
-            dEr[i] = E;
-            dLr[i] = (((kPi * kA0) * j.Ele) * kMe) / (((j.MSHI * j.Zeff) * j.Zeff) * Ltot1);
-        }
-    }
-    if (hw) {
-        for (int64_t t = i; t < rlen; ++t) { hw[t] = 0.0; cum[t] = 0.0; }
-    }
+    if (hw)
+        for (int64_t t = o1 - o + lane; t < rlen; t += 64) entry(t, 0.0, 0.0);
+    if (lane) return;
     int64_t tix = (int64_t)j.shell * out.n + j.ie;
     if (j.type == ROW_INEL) {
         double Sigma, D;
@@ -570,18 +943,13 @@ __global__ void k_row_scan(const RowJob *__restrict__ jobs, int nrows, const int
         else { Sigma = 1.0 / (j.Mass * Ltot1); D = j.Mass * ddEdx; }
         out.L[tix] = Sigma;
         out.dEdx[tix] = D;
-        if (hw)
-            for (int64_t t = 0; t < rlen; ++t) cum[t] = (cum[t] < 1.0e-15) ? 1.0e15 : 1.0 / (j.Mass * cum[t]);
     } else if (j.type == ROW_PHONON) {
-        double Z2M = (j.Zeff * j.Zeff) * j.Mass;
         double Sigma;
         if ((j.Mass < 1.0e-20) || (Ltot1 < 1.0e-15)) Sigma = 1.0e29;
         else Sigma = 1.0 / (Z2M * Ltot1);
         if (Sigma > 1.0e30) Sigma = 1.0e30;
         out.L[j.ie] = Sigma;
         out.dEdx[j.ie] = Z2M * ddEdx;
-        if (hw)
-            for (int64_t t = 0; t < rlen; ++t) cum[t] = (cum[t] < 1.0e-15) ? 1.0e20 : 1.0 / (Z2M * cum[t]);
     } else if (j.type == ROW_SHI) {
         double pre = (1.0 / ((kPi * kA0) * j.Ele)) * j.MSHI;
         // a Brandt-Kitagawa ion carries its charge inside the integrand
@@ -832,6 +1200,22 @@ static int dalloc(T **p, size_t n, std::string &err)
     return 0;
 }
 
+// Entries of the density of states that k_eval follows by their momentum: all
+// of them if the material takes its masses from there, the momenta increase,
+// and the masses are ordinary numbers; else 0 (a search of every momentum).
+static int dos_masses(const HostMat &h, const MatDev &md)
+{
+    if (!md.use_k || md.nk < 1 || md.nk > kMaxDosMass) return 0;
+    const bool metal = h.Egap < 0.2;       // the choice of the uploaded pair
+    const std::vector<double> &k = metal ? h.doskI : h.dosk, &M = metal ? h.dosMI : h.dosM;
+    if ((int)k.size() < md.nk || (int)M.size() < md.nk) return 0;
+    for (int i = 0; i < md.nk; ++i) {
+        if (!(k[i] >= 0.0) || !(M[i] >= 1.0e-6 && M[i] <= 1.0e6)) return 0;
+        if (i && !(k[i] >= k[i - 1])) return 0;
+    }
+    return (k[md.nk - 1] > 0.0 && k[md.nk - 1] < 1.0e300) ? md.nk : 0;
+}
+
 static inline unsigned nblk(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
 
 void free_tables(TableSet &ts)
@@ -990,7 +1374,7 @@ int build_tables(const HostMat &h, const MatDev &md, TableSet &ts, hipStream_t s
     int *d_cnt = nullptr, *d_len = nullptr;
     if (dalloc(&d_jobs, nrows, err) || dalloc(&d_cnt, nrows, err) || dalloc(&d_len, nrows, err)) return TRK_ERR_DEVICE;
     HIP_OK(hipMemcpyAsync(d_jobs, jobs.data(), sizeof(RowJob) * nrows, hipMemcpyHostToDevice, st));
-    k_row_plan<<<nblk(nrows, 64), 64, 0, st>>>(d_jobs, nrows, d_cnt, d_len);
+    k_row_plan<<<nblk(nrows, 4), 256, 0, st>>>(d_jobs, nrows, d_cnt, d_len);
     HIP_OK(hipGetLastError());
     std::vector<int> cnt(nrows), len(nrows);
     HIP_OK(hipMemcpyAsync(cnt.data(), d_cnt, sizeof(int) * nrows, hipMemcpyDeviceToHost, st));
@@ -1004,9 +1388,12 @@ int build_tables(const HostMat &h, const MatDev &md, TableSet &ts, hipStream_t s
         }
 
     // step offsets
-    std::vector<int64_t> step_off(nrows + 1, 0);
-    for (int r = 0; r < nrows; ++r) step_off[r + 1] = step_off[r] + cnt[r];
-    const int64_t nsteps = step_off[nrows];
+    std::vector<int64_t> step_off(nrows + 1, 0), chunk_off(nrows + 1, 0);
+    for (int r = 0; r < nrows; ++r) {
+        step_off[r + 1] = step_off[r] + cnt[r];
+        chunk_off[r + 1] = chunk_off[r] + row_chunks(cnt[r]);
+    }
+    const int64_t nsteps = step_off[nrows], nchunks = chunk_off[nrows];
 
     // row storage per kind: row_off over (shell, ie)
     if (own)
@@ -1042,18 +1429,21 @@ int build_tables(const HostMat &h, const MatDev &md, TableSet &ts, hipStream_t s
     HIP_OK(hipMemcpyAsync(d_doff, td.doff.data(), sizeof(int64_t) * (nsh + 1), hipMemcpyHostToDevice, st));
 
     // nodes and evaluations
-    int64_t *d_step_off = nullptr;
+    int64_t *d_step_off = nullptr, *d_chunk_off = nullptr;
     double *d_Ek = nullptr, *d_dEk = nullptr, *d_f0 = nullptr, *d_fa = nullptr, *d_fb = nullptr;
-    int *d_step_row = nullptr;
-    if (dalloc(&d_step_off, nrows + 1, err) || dalloc(&d_Ek, nsteps, err) || dalloc(&d_dEk, nsteps, err) ||
-        dalloc(&d_f0, nrows, err) || dalloc(&d_fa, nsteps, err) || dalloc(&d_fb, nsteps, err) ||
-        dalloc(&d_step_row, nsteps, err))
+    int *d_chunk_row = nullptr;
+    if (dalloc(&d_step_off, nrows + 1, err) || dalloc(&d_chunk_off, nrows + 1, err) || dalloc(&d_Ek, nsteps, err) ||
+        dalloc(&d_dEk, nsteps, err) || dalloc(&d_f0, nrows, err) || dalloc(&d_fa, nsteps, err) ||
+        dalloc(&d_fb, nsteps, err) || dalloc(&d_chunk_row, nchunks, err))
         return TRK_ERR_DEVICE;
     HIP_OK(hipMemcpyAsync(d_step_off, step_off.data(), sizeof(int64_t) * (nrows + 1), hipMemcpyHostToDevice, st));
-    k_row_nodes<<<nblk(nrows, 64), 64, 0, st>>>(d_jobs, nrows, d_step_off, d_Ek, d_dEk, d_step_row);
+    HIP_OK(hipMemcpyAsync(d_chunk_off, chunk_off.data(), sizeof(int64_t) * (nrows + 1), hipMemcpyHostToDevice, st));
+    k_row_nodes<<<nblk(nrows, 4), 256, 0, st>>>(d_jobs, nrows, d_step_off, d_chunk_off, d_Ek, d_dEk, d_chunk_row);
     HIP_OK(hipGetLastError());
     int64_t npts = nrows + 2 * nsteps;
-    k_eval<<<nblk(npts, 256), 256, 0, st>>>(md, d_jobs, nrows, nsteps, d_Ek, d_dEk, d_step_row, d_f0, d_fa, d_fb);
+    const int dos_n = dos_masses(h, md);
+    k_eval<<<nblk(nchunks, kEvalBlock / kPointsWave), kEvalBlock, sizeof(double) * 3 * dos_n, st>>>(
+        md, d_jobs, d_chunk_row, d_chunk_off, d_step_off, nchunks, d_Ek, d_dEk, d_f0, d_fa, d_fb, dos_n);
     HIP_OK(hipGetLastError());
     ts.dcs_evals = npts;
 
@@ -1069,7 +1459,7 @@ int build_tables(const HostMat &h, const MatDev &md, TableSet &ts, hipStream_t s
     RowOut *d_outs = nullptr;
     if (dalloc(&d_outs, 7, err)) return TRK_ERR_DEVICE;
     HIP_OK(hipMemcpyAsync(d_outs, outs, sizeof(outs), hipMemcpyHostToDevice, st));
-    k_row_scan<<<nblk(nrows, 64), 64, 0, st>>>(d_jobs, nrows, d_step_off, d_Ek, d_dEk, d_f0, d_fa, d_fb, d_outs,
+    k_row_scan<<<nblk(nrows, 4), 256, 0, st>>>(d_jobs, nrows, d_step_off, d_Ek, d_dEk, d_f0, d_fa, d_fb, d_outs,
                                                 td.dE, td.dL, d_doff);
     HIP_OK(hipGetLastError());
 
@@ -1207,7 +1597,7 @@ int build_tables(const HostMat &h, const MatDev &md, TableSet &ts, hipStream_t s
         k_log<<<(unsigned)((m + 127) / 128), 128, 0, st>>>(T[k].lam, m, ts.ln_lam[k]);
         const int64_t nslots = (int64_t)T[k].nsh * T[k].n;
         if (dalloc(&T[k].row_mono, nslots, err)) return TRK_ERR_DEVICE;
-        k_row_mono<<<(unsigned)((nslots + 127) / 128), 128, 0, st>>>(T[k].row_off, nslots, T[k].lam, T[k].row_mono);
+        k_row_mono<<<nblk(nslots, 4), 256, 0, st>>>(T[k].row_off, nslots, T[k].lam, T[k].row_mono);
     }
     HIP_OK(hipGetLastError());
     HIP_OK(hipStreamSynchronize(st));
@@ -1233,7 +1623,7 @@ int build_tables(const HostMat &h, const MatDev &md, TableSet &ts, hipStream_t s
     }
     (void)hipFree(d_jobs); (void)hipFree(d_cnt); (void)hipFree(d_len); (void)hipFree(d_doff);
     (void)hipFree(d_step_off); (void)hipFree(d_Ek); (void)hipFree(d_dEk); (void)hipFree(d_f0);
-    (void)hipFree(d_fa); (void)hipFree(d_fb); (void)hipFree(d_step_row); (void)hipFree(d_outs);
+    (void)hipFree(d_fa); (void)hipFree(d_fb); (void)hipFree(d_chunk_off); (void)hipFree(d_chunk_row); (void)hipFree(d_outs);
     ts.launches = 12;
     ts.build_seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t_start).count();
     return 0;
@@ -1275,7 +1665,7 @@ int refresh_derived(const HostMat &h, TableSet &ts, hipStream_t st, std::string 
         k_log<<<(unsigned)((m + 127) / 128), 128, 0, st>>>(T[k].hw, m, ts.ln_hw[k]);
         k_log<<<(unsigned)((m + 127) / 128), 128, 0, st>>>(T[k].lam, m, ts.ln_lam[k]);
         const int64_t nslots = (int64_t)T[k].nsh * T[k].n;
-        k_row_mono<<<(unsigned)((nslots + 127) / 128), 128, 0, st>>>(T[k].row_off, nslots, T[k].lam, T[k].row_mono);
+        k_row_mono<<<nblk(nslots, 4), 256, 0, st>>>(T[k].row_off, nslots, T[k].lam, T[k].row_mono);
     }
     TableDev &td = T[TRK_TAB_SHI_DIFF];
     HIP_OK(hipMemsetAsync(td.dNonMono, 0, sizeof(int) * nsh, st));
