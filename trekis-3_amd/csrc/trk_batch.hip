@@ -121,20 +121,12 @@ static int balloc(trk_batch *b, T **p, size_t n)
 
 static int batch_alloc_list(trk_batch *b, PList &l, int cap, int hole)
 {
-    const size_t n = (size_t)(cap > 0 ? cap : 1);
-    double **dp[] = {&l.E, &l.t0, &l.tn, &l.X, &l.Y, &l.Z, &l.L, &l.th, &l.ph};
-    for (double **p : dp) if (balloc(b, p, n)) return TRK_ERR_DEVICE;
-    if (hole) {
-        if (balloc(b, &l.Ehkin, n) || balloc(b, &l.Mass, n) || balloc(b, &l.sh, n)) return TRK_ERR_DEVICE;
-    }
-    if (balloc(b, &l.id, n) || balloc(b, &l.nd, n) || balloc(b, &l.ne, n) || balloc(b, &l.iter, n)) return TRK_ERR_DEVICE;
-    return 0;
+    return balloc(b, (unsigned char **)&l.w, list_bytes((size_t)(cap > 0 ? cap : 1), hole));
 }
 
 static void batch_free_list(PList &l)
 {
-    void *ps[] = {l.E, l.t0, l.tn, l.X, l.Y, l.Z, l.L, l.th, l.ph, l.Ehkin, l.Mass, l.sh, l.id, l.nd, l.ne, l.iter};
-    for (void *p : ps) if (p) (void)hipFree(p);
+    if (l.w) (void)hipFree(l.w);
     l = PList{};
 }
 

@@ -11,12 +11,18 @@
 namespace trk {
 
 // ---------------------------------------------------------------- layouts
-struct PList {            // SoA particle list
-    double *E, *t0, *tn, *X, *Y, *Z, *L, *th, *ph, *Ehkin, *Mass;
-    int *sh;
-    uint64_t *id;
-    uint32_t *nd, *ne, *iter;
+// A particle list: one record of 4-byte words per particle, back to back.  A
+// wave appends 64 records as one contiguous range, a lane that takes a single
+// particle touches one or two cache lines instead of one per field, and the
+// event code keeps one address per list in scalar registers.
+struct PList {
+    uint32_t *w;
 };
+
+// Bytes allocated per particle: the FP64 record without and with the fields
+// of holes and ions (the mixed path's records are shorter).
+constexpr size_t kRecordBytes = 92, kHoleRecordBytes = 112;
+inline size_t list_bytes(size_t n, int hole) { return n * (hole ? kHoleRecordBytes : kRecordBytes); }
 
 struct Tally {            // fixed-point difference arrays, replicated R times
     int Nt, NR, nsh, R;

@@ -300,28 +300,13 @@ struct McState {
 
 static int alloc_list(trk_ctx *c, PList &l, int cap, int hole)
 {
-    size_t n = (size_t)cap;
-    double **dp[] = {&l.E, &l.t0, &l.tn, &l.X, &l.Y, &l.Z, &l.L, &l.th, &l.ph};
-    for (double **p : dp) HIPC(hipMalloc((void **)p, n * sizeof(double)));
-    if (hole) {
-        HIPC(hipMalloc((void **)&l.Ehkin, n * sizeof(double)));
-        HIPC(hipMalloc((void **)&l.Mass, n * sizeof(double)));
-        HIPC(hipMalloc((void **)&l.sh, n * sizeof(int)));
-    } else {
-        l.Ehkin = l.Mass = nullptr;
-        l.sh = nullptr;
-    }
-    HIPC(hipMalloc((void **)&l.id, n * sizeof(uint64_t)));
-    HIPC(hipMalloc((void **)&l.nd, n * sizeof(uint32_t)));
-    HIPC(hipMalloc((void **)&l.ne, n * sizeof(uint32_t)));
-    HIPC(hipMalloc((void **)&l.iter, n * sizeof(uint32_t)));
+    HIPC(hipMalloc((void **)&l.w, list_bytes((size_t)cap, hole)));
     return 0;
 }
 
 static void free_list(PList &l)
 {
-    void *ps[] = {l.E, l.t0, l.tn, l.X, l.Y, l.Z, l.L, l.th, l.ph, l.Ehkin, l.Mass, l.sh, l.id, l.nd, l.ne, l.iter};
-    for (void *p : ps) if (p) (void)hipFree(p);
+    if (l.w) (void)hipFree(l.w);
     l = PList{};
 }
 
@@ -1135,12 +1120,7 @@ struct Carver {
 
 static void carve_list(Carver &cv, PList &l, size_t n, int hole)
 {
-    l.E = cv.take<double>(n); l.t0 = cv.take<double>(n); l.tn = cv.take<double>(n);
-    l.X = cv.take<double>(n); l.Y = cv.take<double>(n); l.Z = cv.take<double>(n);
-    l.L = cv.take<double>(n); l.th = cv.take<double>(n); l.ph = cv.take<double>(n);
-    if (hole) { l.Ehkin = cv.take<double>(n); l.Mass = cv.take<double>(n); l.sh = cv.take<int>(n); }
-    else { l.Ehkin = l.Mass = nullptr; l.sh = nullptr; }
-    l.id = cv.take<uint64_t>(n); l.nd = cv.take<uint32_t>(n); l.ne = cv.take<uint32_t>(n); l.iter = cv.take<uint32_t>(n);
+    l.w = (uint32_t *)cv.take<unsigned char>(list_bytes(n, hole));
 }
 
 // doubles of the caller's Out_* arrays the device finalize stages
