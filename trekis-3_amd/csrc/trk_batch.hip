@@ -177,48 +177,6 @@ __global__ void k_elat_to_i128(unsigned long long *Elat, int64_t ncell)
     if (i < ncell) i128_store(Elat + 2 * i, fx_read(Elat + 2 * i));
 }
 
-// Running sum over the time nodes of the difference arrays of every tally
-// plane (one plane per impact), from the split fixed-point form of the
-// energies to 128-bit integers, as the replica sum and time prefix of a
-// single run leave them (the lattice energy is converted by k_elat_to_i128).
-__global__ void k_time_prefix_planes(Tally T)
-{
-    const int NR = T.NR, Nt = T.Nt, nsh = T.nsh, R = T.R;
-    const int64_t per = 2 * (int64_t)NR + (int64_t)NR * nsh;
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= per * R) return;
-    const int64_t r = t / per, q = t % per;
-    const size_t plane = (size_t)Nt * NR, base = (size_t)r * plane;
-    if (q < 2 * NR) {
-        const int j = (int)(q % NR);
-        unsigned long long *cnt = (q < NR) ? T.cnt_e : T.cnt_p;
-        unsigned long long *en = (q < NR) ? T.E_e : T.E_p;
-        long long rc = 0;
-        __int128 re = 0;
-        for (int i = 0; i < Nt; ++i) {
-            const size_t a = base + (size_t)i * NR + j;
-            rc += (long long)cnt[a];
-            re += fx_read(en + 2 * a);
-            cnt[a] = (unsigned long long)rc;
-            i128_store(en + 2 * a, re);
-        }
-    } else {
-        const int64_t u = q - 2 * NR;
-        const int j = (int)(u / nsh), sh = (int)(u % nsh);
-        long long rc = 0;
-        __int128 rE = 0, rK = 0;
-        for (int i = 0; i < Nt; ++i) {
-            const size_t a = (base + (size_t)i * NR + j) * nsh + sh;
-            rc += (long long)T.cnt_h[a];
-            rE += fx_read(T.E_h + 2 * a);
-            rK += fx_read(T.Ek_h + 2 * a);
-            T.cnt_h[a] = (unsigned long long)rc;
-            i128_store(T.E_h + 2 * a, rE);
-            i128_store(T.Ek_h + 2 * a, rK);
-        }
-    }
-}
-
 static void batch_free(trk_batch *b)
 {
     if (!b) return;
@@ -365,14 +323,14 @@ static int batch_capture(trk_batch *b)
     else if (b->mixed) mx::k_batch<false><<<nblk, b->block, b->lds_bytes, st>>>(b->d_ctl, G);
     else if (b->all_staged) fp64::k_batch<true><<<nblk, b->block, b->lds_bytes, st>>>(b->d_ctl, G);
     else fp64::k_batch<false><<<nblk, b->block, b->lds_bytes, st>>>(b->d_ctl, G);
+    hipError_t te = hipSuccess;
     for (int g = 0; g < G; ++g) {
         const Tally &T = b->groups[g].T;
-        const int64_t n = (2 * (int64_t)T.NR + (int64_t)T.NR * T.nsh) * T.R;
-        k_time_prefix_planes<<<(unsigned)((n + 63) / 64), 64, 0, st>>>(T);
+        if (te == hipSuccess) te = launch_time_prefix(T, T.R, true, st);
         const int64_t nc = (int64_t)T.R * T.Nt * T.NR;
         k_elat_to_i128<<<(unsigned)((nc + 255) / 256), 256, 0, st>>>(T.Elat, nc);
     }
-    const hipError_t le = hipGetLastError();
+    const hipError_t ge = hipGetLastError(), le = (te != hipSuccess) ? te : ge;
     hipGraph_t graph = nullptr;
     const hipError_t ce = hipStreamEndCapture(st, &graph);
     if (le != hipSuccess) { if (graph) (void)hipGraphDestroy(graph); return berr(b, TRK_ERR_DEVICE, "launch in capture: %s", hipGetErrorString(le)); }

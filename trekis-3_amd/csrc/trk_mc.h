@@ -249,6 +249,9 @@ static inline int ion_round_events(double pairs, int n_ions, int cap, int round_
 }
 // BEB shells or the Delta-CDF model: the transport kernel's general instantiation
 bool uses_general_kernel(const HostMat &h);
+// The running sums over time of the tally planes of T, energies as split words
+// (split) or as 128-bit integers.
+hipError_t launch_time_prefix(const Tally &T, int planes, bool split, hipStream_t st);
 // One tally plane converted and added into the caller's Out_* arrays (trk_mc.hip).
 int finish_tallies_host(trk_ctx *c, const Tally &T, int plane_index, const double *Out_V, int NR, trk_tallies *out,
                         hipStream_t st);
