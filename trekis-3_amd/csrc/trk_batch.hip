@@ -61,7 +61,8 @@ struct trk_batch {
     bool mixed = false;
     int NR = 0;
     std::vector<double> R, V;
-    double *d_R = nullptr;
+    double *d_R = nullptr, *d_V = nullptr;
+    trk::FinStage fin[2];                 // finished tallies on their way to the caller
     trk::IonDev *d_ions = nullptr;
     int *d_plane_of = nullptr;            // each impact's tally plane in its group
     std::vector<int> plane_of, group_of;
@@ -191,7 +192,8 @@ static void batch_free(trk_batch *b)
         for (void *p : ps) if (p) (void)hipFree(p);
     }
     b->groups.clear();
-    void *ps[] = {b->d_R, b->d_ions, b->d_plane_of, b->d_ctl, b->d_overflow, b->d_counters, b->d_trace, b->d_trace_n};
+    for (FinStage &f : b->fin) f.release();
+    void *ps[] = {b->d_R, b->d_V, b->d_ions, b->d_plane_of, b->d_ctl, b->d_overflow, b->d_counters, b->d_trace, b->d_trace_n};
     for (void *p : ps) if (p) (void)hipFree(p);
     if (b->ev0) (void)hipEventDestroy(b->ev0);
     if (b->ev1) (void)hipEventDestroy(b->ev1);
@@ -398,16 +400,28 @@ static int batch_launch(trk_batch *b, uint64_t seed, int64_t first_iter, trk_tal
     return outs ? batch_fetch(b, outs) : 0;
 }
 
-// The host tallies of every impact of the last run, from its finished planes.
+// The host tallies of every impact of the last run, from its finished planes:
+// the device prepares and copies one impact's while the host adds the one
+// before.
 static int batch_fetch(trk_batch *b, trk_tallies *const *outs)
 {
     const int n = (int)b->impacts.size();
-    for (int i = 0; i < n; ++i) {
-        if (!outs[i]) continue;
-        trk_ctx *c = b->impacts[i];
-        const Tally &T = b->groups[b->group_of[i]].T;
-        const int rc = finish_tallies_host(c, T, b->plane_of[i], b->V.data(), b->NR, outs[i], b->stream);
-        if (rc) return berr(b, rc, "tallies of impact %d: %s", i, c->err.c_str());
+    int before = -1, half = 0;
+    for (int i = 0; i <= n; ++i) {
+        if (i < n && !outs[i]) continue;
+        if (i < n) {
+            trk_ctx *c = b->impacts[i];
+            const Tally &T = b->groups[b->group_of[i]].T;
+            const int rc = finish_begin(c, b->fin[half], T, b->plane_of[i], b->d_V, b->NR, outs[i], b->stream);
+            if (rc) return berr(b, rc, "tallies of impact %d: %s", i, c->err.c_str());
+        }
+        if (before >= 0) {
+            trk_ctx *c = b->impacts[before];
+            const int rc = finish_end(c, b->fin[1 - half], b->NR, outs[before]);
+            if (rc) return berr(b, rc, "tallies of impact %d: %s", before, c->err.c_str());
+        }
+        before = i;
+        half = 1 - half;
     }
     return 0;
 }
@@ -521,8 +535,9 @@ int trk_batch_create(trk_ctx *const *impacts, int32_t n, const double *Out_R, co
     b->R.assign(Out_R, Out_R + NR);
     b->V.assign(Out_V, Out_V + NR);
     b->capacity = capacity > 0 ? capacity : (1 << 22);
-    if (balloc(b, &b->d_R, NR)) return TRK_ERR_DEVICE;
+    if (balloc(b, &b->d_R, NR) || balloc(b, &b->d_V, NR)) return TRK_ERR_DEVICE;
     BHIP(hipMemcpy(b->d_R, Out_R, sizeof(double) * NR, hipMemcpyHostToDevice));
+    BHIP(hipMemcpy(b->d_V, Out_V, sizeof(double) * NR, hipMemcpyHostToDevice));
     // the control block and, after it, kMaxGroups ion counts of the capture
     if (balloc(b, (char **)&b->d_ctl, 2 * sizeof(BatchCtl) + sizeof(int) * kMaxGroups)) return TRK_ERR_DEVICE;
     if (balloc(b, &b->d_overflow, 1) || balloc(b, &b->d_counters, 16)) return TRK_ERR_DEVICE;

@@ -252,9 +252,28 @@ bool uses_general_kernel(const HostMat &h);
 // The running sums over time of the tally planes of T, energies as split words
 // (split) or as 128-bit integers.
 hipError_t launch_time_prefix(const Tally &T, int planes, bool split, hipStream_t st);
-// One tally plane converted and added into the caller's Out_* arrays (trk_mc.hip).
-int finish_tallies_host(trk_ctx *c, const Tally &T, int plane_index, const double *Out_V, int NR, trk_tallies *out,
-                        hipStream_t st);
+// Staging of one plane's finished tallies: device and page-locked host values,
+// kept by the object (context or batch) whose runs use it and grown to the
+// largest plane it was asked for.
+struct FinStage {
+    double *dev = nullptr, *pin = nullptr;
+    unsigned long long *node_sums = nullptr;   // [Nt][4]: lattice energy of the node, the rest of tot_E
+    hipEvent_t done = nullptr;                 // the values are in pin
+    size_t n = 0, node_n = 0;
+    int grow(size_t values, size_t nodes);
+    void release();
+};
+// values already on the device that a run adds to another of the caller's arrays
+struct FinExtra {
+    const double *dev;
+    double *dst;
+    size_t n;
+};
+// One tally plane converted on the device and copied to the stage, and then
+// added into the caller's Out_* arrays (trk_mc.hip).  d_V: Out_V on the device.
+int finish_begin(trk_ctx *c, FinStage &fs, const Tally &T, int plane_index, const double *d_V, int NR,
+                 const trk_tallies *out, hipStream_t st, const std::vector<FinExtra> *extra = nullptr);
+int finish_end(trk_ctx *c, FinStage &fs, int NR, trk_tallies *out, const std::vector<FinExtra> *extra = nullptr);
 
 // 128-bit tally words: (low, high) 64-bit halves of an exact integer
 TRK_DEV __int128 fx_read(const unsigned long long *p)
