@@ -206,8 +206,11 @@ static int batch_shape(trk_batch *b)
 {
     const void *kt = b->mixed ? (b->all_staged ? (const void *)mx::k_batch<true> : (const void *)mx::k_batch<false>)
                               : (b->all_staged ? (const void *)fp64::k_batch<true> : (const void *)fp64::k_batch<false>);
+    const void *ki = b->mixed ? (b->all_staged ? (const void *)mx::k_batch_ions<true> : (const void *)mx::k_batch_ions<false>)
+                              : (b->all_staged ? (const void *)fp64::k_batch_ions<true> : (const void *)fp64::k_batch_ions<false>);
     if (b->lds_bytes > 65536)
-        BHIP(hipFuncSetAttribute(kt, hipFuncAttributeMaxDynamicSharedMemorySize, (int)b->lds_bytes));
+        for (const void *k : {kt, ki})
+            BHIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)b->lds_bytes));
     int per_cu = 0;
     BHIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kt, b->block, b->lds_bytes));
     if (per_cu < 1) return berr(b, TRK_ERR_CAPACITY, "a %d-thread batch workgroup with %zu bytes of LDS does not fit a CU",
@@ -320,6 +323,21 @@ static int batch_capture(trk_batch *b)
         if (b->mixed) mx::k_ion_init_batch<<<(nb + 63) / 64, 64, 0, st>>>(g, nb, b->groups[g].d_idx);
         else fp64::k_ion_init_batch<<<(nb + 63) / 64, 64, 0, st>>>(g, nb, b->groups[g].d_idx);
     }
+    // the CUs are shared out by the groups' numbers of ions
+    BatchIons bi{};
+    for (int g = 0; g < G; ++g) {
+        const int64_t n = nions[g], all = (int64_t)b->impacts.size();
+        int64_t share = (n * b->ncu + all - 1) / all;
+        if (share < 1) share = 1;
+        bi.waves[g] = ion_waves(n, share);
+        const int64_t need = (n + bi.waves[g] - 1) / bi.waves[g];
+        bi.first[g + 1] = bi.first[g] + (int)(need < share ? need : share);
+    }
+    const unsigned nion = (unsigned)bi.first[G];
+    if (b->mixed && b->all_staged) mx::k_batch_ions<true><<<nion, kIonBlock, b->lds_bytes, st>>>(bi, G);
+    else if (b->mixed) mx::k_batch_ions<false><<<nion, kIonBlock, b->lds_bytes, st>>>(bi, G);
+    else if (b->all_staged) fp64::k_batch_ions<true><<<nion, kIonBlock, b->lds_bytes, st>>>(bi, G);
+    else fp64::k_batch_ions<false><<<nion, kIonBlock, b->lds_bytes, st>>>(bi, G);
     const unsigned nblk = (unsigned)b->blocks;
     if (b->mixed && b->all_staged) mx::k_batch<true><<<nblk, b->block, b->lds_bytes, st>>>(b->d_ctl, G);
     else if (b->mixed) mx::k_batch<false><<<nblk, b->block, b->lds_bytes, st>>>(b->d_ctl, G);

@@ -212,6 +212,20 @@ constexpr int kSparseWaves = 4;
 // Workgroup of the ion kernel: 8 waves, each with one ion, 2 per SIMD.
 constexpr int kIonBlock = 512;
 
+// The ions' workgroups of a batch: those of group g start at first[g], each
+// with waves[g] ions at a time.
+struct BatchIons {
+    int first[kMaxGroups + 1], waves[kMaxGroups];
+};
+
+// Waves per workgroup for n ions and at most `groups` workgroups: one ion per CU
+// while there are few, up to the workgroup's eight.
+inline int ion_waves(int64_t n, int64_t groups)
+{
+    const int64_t per = (n + groups - 1) / groups;
+    return (int)(per < kIonBlock / 64 ? per : kIonBlock / 64);
+}
+
 // The event code is compiled twice, into namespaces fp64 (deterministic
 // FP64, replays the oracle bit for bit) and mx (mixed precision); these are
 // the kernels the host driver launches from each.
@@ -222,6 +236,7 @@ constexpr int kIonBlock = 512;
     __global__ void k_shi_consts(IonDev iv, const double *Ip, int nsh, int *sd_M, double *sd_c); \
     __global__ void k_shi_buckets(IonDev iv, int nsh, const int *sd_M, const double *sd_c, int *sd_bk); \
     template <bool kAll> __global__ void k_batch(BatchCtl *ctl, int n_groups); \
+    template <bool kAll> __global__ void k_batch_ions(BatchIons bi, int n_groups); \
     __global__ void k_ion_init_batch(int g, int nb, const int *idx);        \
     hipError_t batch_upload(const McDev *mc, int n_groups, hipStream_t st);
 namespace fp64 { TRK_MC_KERNELS }

@@ -1078,10 +1078,7 @@ static int run_rounds(trk_ctx *c, McState *s, int64_t nmc, uint64_t seed, int64_
             HIPC(hipMemsetAsync(d.cursor, 0, 2 * sizeof(int), st));
             const size_t lds = s->lds_bytes;
             if (nin[K_ION] > 0) {
-                // one wave per ion: one per CU while there are few, up to the
-                // workgroup's eight
-                const int64_t per = (nin[K_ION] + s->ncu - 1) / s->ncu;
-                const int waves = (int)(per < kIonBlock / 64 ? per : kIonBlock / 64);
+                const int waves = ion_waves(nin[K_ION], s->ncu);
                 const int64_t need = (nin[K_ION] + waves - 1) / waves;
                 const unsigned gi = (unsigned)(need < s->ncu ? need : s->ncu);
                 if (c->prof) HIPC(hipEventRecord(c->pe[2], st));

@@ -9,6 +9,8 @@ namespace mx {
 #undef TRK_MX
 #undef TRK_PART
 
+template __global__ void k_batch_ions<true>(BatchIons bi, int n_groups);
+template __global__ void k_batch_ions<false>(BatchIons bi, int n_groups);
 template __global__ void k_batch<true>(BatchCtl *ctl, int n_groups);
 template __global__ void k_batch<false>(BatchCtl *ctl, int n_groups);
 }  // namespace mx
