@@ -190,6 +190,23 @@ constexpr int kWaveNodes = 3;
 // the cost of kRoundEvents events instead of the longest history.
 constexpr uint32_t kRoundEvents = 512;
 
+// The budget of a round of n particles on `lanes` lanes.  A round lasts until
+// its longest history has used the budget, and children wait for its end:
+// with few particles a lane, a smaller budget starts them earlier.  Below 128
+// the rounds' own cost (a launch, the staging, a read of the counts) shows;
+// with eight budgets' worth of particles a lane the end of a round does not.
+// Budgets of 512 against this rule: 25 oxide iterations 16.7 -> 11.9 ms, 1000
+// of them in FP64 240 -> 217, the track target 42 -> 37; 128 for every round
+// made 4001 oxide iterations slower (430 -> 490).  free: only where the lists are
+// long (the ions may run on beyond the budget), since particles that wait
+// between rounds take room in them.
+TRK_HD int round_budget(long long n, long long lanes, int budget, bool free)
+{
+    const long long b = 8 * n / lanes;
+    if (!free || b >= budget) return budget;
+    return b > 128 ? (int)b : (budget < 128 ? budget : 128);
+}
+
 extern __shared__ double lds_tab[];
 
 // The sources a path's kernels are spread over (TRK_PART): the transport of

@@ -1095,6 +1095,7 @@ static int run_rounds(trk_ctx *c, McState *s, int64_t nmc, uint64_t seed, int64_
                 int64_t nblk = (nthr + tb - 1) / tb;
                 int tbl = tb;             // threads per workgroup of this launch
                 d.lane_cap = 64;
+                d.round_events = round_budget(nthr, s->max_blocks * tb, (int)kRoundEvents, d.ion_events > (int)kRoundEvents);
                 if (nthr < 64 * kSparseWaves * s->max_blocks) {
                     // few particles (the last rounds of a large run, all of
                     // a small one): as many waves as there are SIMDs, with as
