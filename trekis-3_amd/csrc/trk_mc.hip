@@ -10,21 +10,22 @@
 //    a thread owns one particle and runs all of its events.  Each particle has
 //    its own counter-based random stream, so the order in which the GPU
 //    visits particles does not change any history.
-//  * Particles are processed in generations.  Generation 0 is the ion of every
-//    iteration of a batch (one thread per iteration); the electron/hole pairs
-//    it creates form generation 1; the secondaries of generation g form g+1.
-//    Children are appended with one wave-aggregated atomic per allocation, and
-//    pairs are stored SoA in separate electron and hole lists so that a wave
-//    holds particles of one kind.
+//  * Particles are processed in rounds: the electrons, holes and photons of a
+//    round's lists take up to a budget of events each (round_budget), and
+//    what they make, with what they leave unfinished, forms the next round's
+//    lists.  The ions are run by whole waves (k_ions), all of their collisions
+//    in the first round where the lists are long enough.  Children are
+//    appended with one wave-aggregated atomic per list, as records, electrons
+//    and holes apart so that a wave holds particles of one kind.
 //  * Snapshot tallies (Calculated_statistics, MC:881-1110) are not taken by
 //    scanning all particles at every time node.  A particle's state is
 //    constant between two of its events, so its contribution to the nodes
 //    that fall in that interval is added to difference arrays over time
 //    (one add at the first node, one subtraction after the last); a moving
-//    particle adds one range per radial bin it crosses.  The host prefix-sums
-//    the time axis once per run.  Adds are integer atomics on split fixed-point
-//    accumulators (2^-40 eV resolution), which makes every tally independent
-//    of the order of the adds and hence deterministic.
+//    particle adds one range per radial bin it crosses.  The running sums
+//    along the time axis are taken once per run.  Adds are integer atomics on
+//    split fixed-point accumulators (2^-40 eV resolution), which makes every
+//    tally independent of the order of the adds and hence deterministic.
 #include <hip/hip_runtime.h>
 #include <chrono>
 #include <cstdio>
@@ -769,8 +770,8 @@ int finish_end(trk_ctx *c, FinStage &fs, int NR, trk_tallies *out, const std::ve
     return 0;
 }
 
-// Each generation is the set of particles born in the previous one; a chain of
-// ionisations is at most a few hundred long.
+// Rounds of one batch: a particle of kMaxEvents events at the smallest budget
+// (128) takes half of these.
 constexpr int kMaxGenerations = 1 << 16;
 
 // The ion's expected ionisations over the layer.
@@ -781,7 +782,7 @@ static double ion_collisions(const trk_ctx *c)
 }
 
 // Iterations per batch: the ion's expected ionisations times the pairs each
-// makes must fit one generation's lists.
+// makes must fit one round's lists.
 static int64_t batch_size(const trk_ctx *c, int cap, int64_t nmc)
 {
     const double est_pairs = ion_collisions(c);
