@@ -292,6 +292,7 @@ struct FinStage {
     unsigned long long *node_sums = nullptr;   // [Nt][4]: lattice energy of the node, the rest of tot_E
     hipEvent_t done = nullptr;                 // the values are in pin
     size_t n = 0, node_n = 0;
+    bool locked = false;                       // pin is page-locked
     int grow(size_t values, size_t nodes);
     void release();
 };

@@ -691,11 +691,21 @@ int FinStage::grow(size_t values, size_t nodes)
     release();
     if (hipMalloc((void **)&dev, (values ? values : 1) * sizeof(double)) != hipSuccess ||
         hipMalloc((void **)&node_sums, (nodes ? nodes : 1) * 4 * sizeof(unsigned long long)) != hipSuccess ||
-        hipHostMalloc((void **)&pin, (values ? values : 1) * sizeof(double), hipHostMallocDefault) != hipSuccess ||
         hipEventCreateWithFlags(&done, hipEventDisableTiming) != hipSuccess) {
         (void)hipGetLastError();
         release();
         return 1;
+    }
+    // where no memory can be locked, ordinary memory does (slower)
+    const size_t bytes = (values ? values : 1) * sizeof(double);
+    locked = hipHostMalloc((void **)&pin, bytes, hipHostMallocDefault) == hipSuccess;
+    if (!locked) {
+        (void)hipGetLastError();
+        pin = (double *)std::malloc(bytes);
+        if (!pin) {
+            release();
+            return 1;
+        }
     }
     n = values;
     node_n = nodes;
@@ -706,7 +716,8 @@ void FinStage::release()
 {
     if (dev) (void)hipFree(dev);
     if (node_sums) (void)hipFree(node_sums);
-    if (pin) (void)hipHostFree(pin);
+    if (pin && locked) (void)hipHostFree(pin);
+    else std::free(pin);
     if (done) (void)hipEventDestroy(done);
     dev = pin = nullptr;
     node_sums = nullptr;
