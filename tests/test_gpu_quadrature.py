@@ -66,3 +66,22 @@ def test_loop_forms_agree(name, n, quadrature):
     for k in a:
         for x, y in zip(a[k], b[k]):
             assert np.array_equal(x, y, equal_nan=True), (k, np.flatnonzero(x != y)[:5])
+
+
+# an immobile hole given as an infinite mass: its momentum limits are infinite
+# or NaN, every hole integral is empty, and the tables are the oracle's
+def test_infinite_hole_mass_leaves_empty_integrals():
+    from oracle import Oracle
+    mat, ion, opt, run = tg.config_material("test_metal")        # electron masses from the density of states
+    mat.hole_mass = float("inf")
+    mat.prepare(tg.load_library())
+    say("[quadrature] test_metal, infinite hole mass")
+    ctx = tg.Context(mat, ion, opt)
+    ctx.build_tables()
+    orc = Oracle(mat, ion, opt)
+    orc.build_tables(8)
+    for kind in (abi.TAB_E_INEL, abi.TAB_H_INEL, abi.TAB_E_EL, abi.TAB_H_EL):
+        for s in [0] if kind in (abi.TAB_E_EL, abi.TAB_H_EL) else range(sum(mat.n_shells)):
+            for x, y in zip(ctx.table(kind, s), orc.table(kind, s)):
+                assert np.array_equal(x, y, equal_nan=True), (kind, s)
+    assert (ctx.table(abi.TAB_H_INEL, 0)[1] >= 1e15).all()

@@ -227,7 +227,10 @@ TRK_DEV double q_simpson(const OscSpan &o, const DosMass &dm, double w, double c
             }
         }
     };
-    if (kDos) {
+    // An empty range (qmin not below qmax) may come with limits that are not
+    // finite, as an infinite hole mass gives: no look then, interval would
+    // never pass an infinite momentum.
+    if (kDos && qmin < qmax) {
         const double v = qmin * rootE;
         int lo = -1, hi = dm.nk;      // k[lo] <= v < k[hi]
         while (hi - lo > 1) {
