@@ -14,8 +14,8 @@
  * Draw n of a particle uses block n>>1 of its stream:
  *   ctr = {n>>1, id_lo, id_hi, iteration}, key = {seed_lo, seed_hi}
  * and takes words (0,1) for even n, (2,3) for odd n, combined into a 53-bit
- * integer u; the value is (u + 0.5) * 2^-53, which lies strictly inside (0,1)
- * so -log(RN) is always finite.
+ * integer u; the value is (u + 0.5) * 2^-53, which is never 0, so -log(RN) is
+ * always finite.  It is 1 for u = 2^53 - 1 alone, where u + 0.5 rounds up.
  */
 #ifndef TRK_PHILOX_H
 #define TRK_PHILOX_H
@@ -59,7 +59,7 @@ TRK_RFN trk_u32x4 trk_philox4x32_10(trk_u32x4 c, uint32_t k0, uint32_t k1)
     return c;
 }
 
-/* Uniform double in (0,1) for draw `n` of particle `id` in iteration `iter`. */
+/* Uniform double in (0,1] for draw `n` of particle `id` in iteration `iter`. */
 TRK_RFN double trk_uniform(uint64_t seed, uint64_t id, uint32_t iter, uint32_t n)
 {
     trk_u32x4 c;

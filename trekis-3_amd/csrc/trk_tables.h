@@ -6,6 +6,7 @@
 #include <string>
 #include "trk_dev_common.h"
 #include "trk_dsf.h"
+#include "trk_rules.h"
 
 namespace trk {
 
@@ -36,11 +37,6 @@ struct MatDev {
 };
 
 // One table kind on the device.  Per-shell arrays are shell-major [nsh][n].
-// The ion's energy-transfer draw RN in [b/kShiBuckets, (b+1)/kShiBuckets)
-// finds its entry of a shell's inverse-path row between the entries that
-// the bucket's two ends find (k_shi_buckets).
-constexpr int kShiBuckets = 64;
-
 struct TableDev {
     int n = 0;
     int nsh = 0;
