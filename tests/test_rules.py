@@ -33,3 +33,25 @@ def test_bucket_of_a_draw_stays_in_its_row(tmp_path):
     assert rows[4][0] == 1.0
     for RN, b, n in rows:
         assert 0 <= b < n and b / n <= RN <= (b + 1) / n
+
+
+def test_transport_shape_uses_the_whole_gpu(tmp_path):
+    """Every particle of a round fits its launch's lanes or is taken later by a
+    full grid; no launch has more workgroups or threads than may be resident;
+    and from 64 particles per SIMD on, the launch has a workgroup on at least
+    four fifths of the CUs, with the waves spread evenly."""
+    for cus, full in ((256, 768), (304, 768), (80, 512)):
+        edges = [64 * 4 * cus, full * cus]
+        ns = [1, 2, 3, 63, 64, 65, 4 * cus, 4 * cus + 1] + [e + d for e in edges for d in (-65, -64, -1, 0, 1, 64, 65)]
+        ns += [int(64 * 4 * cus * 1.03 ** k) for k in range(60)] + [10 ** 7, 10 ** 9 + 7]
+        rows = evaluate(tmp_path, "for (int64_t n : {%s}) {\nconst TransportShape s = transport_shape(n, %d, %d);\n"
+                        'printf("%%lld %%lld %%d %%d\\n", (long long)n, (long long)s.blocks, s.threads, s.lane_cap);\n}'
+                        % (", ".join(f"(int64_t){n}" for n in ns), cus, full))
+        for n, blocks, threads, cap in rows:
+            assert 1 <= blocks <= cus and threads % 64 == 0 and 64 <= threads <= full and 1 <= cap <= 64
+            waves = threads / 64
+            assert blocks * waves * cap >= min(n, full * cus), n
+            if n >= 64 * 4 * cus:
+                # one wave less per workgroup would not do, so at most a fifth of the CUs has none
+                assert blocks >= 0.8 * cus, (n, blocks)
+                assert (waves - 1) * 64 * cus < n, (n, waves)

@@ -223,9 +223,6 @@ extern __shared__ double lds_tab[];
 constexpr int kTransportBlockFp64 = 768;
 constexpr int kTransportBlockMx = 768;
 
-// Waves per workgroup (one per SIMD) of a round with few particles.
-constexpr int kSparseWaves = 4;
-
 // Workgroup of the ion kernel: 8 waves, each with one ion, 2 per SIMD.
 constexpr int kIonBlock = 512;
 

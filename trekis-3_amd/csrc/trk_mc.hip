@@ -1104,24 +1104,12 @@ static int run_rounds(trk_ctx *c, McState *s, int64_t nmc, uint64_t seed, int64_
             }
             if (nthr > 0) {
                 const int tb = mixed ? kTransportBlockMx : kTransportBlockFp64;
-                int64_t nblk = (nthr + tb - 1) / tb;
-                int tbl = tb;             // threads per workgroup of this launch
-                d.lane_cap = 64;
+                const TransportShape sh = transport_shape(nthr, s->max_blocks, tb);
+                const int tbl = sh.threads;
+                d.lane_cap = sh.lane_cap;
                 d.round_events = round_budget(nthr, s->max_blocks * tb, (int)kRoundEvents, d.ion_events > (int)kRoundEvents);
-                if (nthr < 64 * kSparseWaves * s->max_blocks) {
-                    // few particles (the last rounds of a large run, all of
-                    // a small one): as many waves as there are SIMDs, with as
-                    // few particles each as that gives; a wave runs each
-                    // category its particles want in turn, so a lone history
-                    // goes faster the fewer share its wave
-                    tbl = 64 * kSparseWaves;
-                    d.lane_cap = (int)((nthr + kSparseWaves * s->max_blocks - 1) / (kSparseWaves * s->max_blocks));
-                    const int64_t per = (int64_t)kSparseWaves * d.lane_cap;
-                    nblk = (nthr + per - 1) / per;
-                }
-                if (nblk > s->max_blocks) nblk = s->max_blocks;
                 if (c->prof) HIPC(hipEventRecord(c->pe[0], st));
-                const unsigned g = (unsigned)nblk;
+                const unsigned g = (unsigned)sh.blocks;
                 if (general) {
                     if (mixed && s->all_staged) mx::k_transport<true, true><<<g, tbl, lds, st>>>(d);
                     else if (mixed) mx::k_transport<false, true><<<g, tbl, lds, st>>>(d);
