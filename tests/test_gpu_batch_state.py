@@ -1,0 +1,44 @@
+"""What a batch keeps from one run to the next: after a run that fails there
+are no tallies to fetch, and a later good run gives its own again."""
+import numpy as np
+import pytest
+
+import trekis_gpu as tg
+from trekis_gpu.batch import Batch, IonContext
+
+from gpu_helpers import say
+
+pytestmark = pytest.mark.gpu
+
+
+def _impact(name, ion_of=None):
+    """(ion context, run values) on a target; ion_of: (Z, mass, MeV/u)"""
+    mat, ion, opt, run = tg.config_material(name)
+    mat.prepare(tg.load_library())
+    ctx = tg.Context(mat, ion, opt)
+    ctx.build_tables()
+    if ion_of:
+        Z, M, E = ion_of
+        ion.Zat, ion.Mass, ion.E = Z, M, E * 1e6 * M
+    c = IonContext(ctx, ion)
+    c.build_tables()
+    return c, run
+
+
+def test_no_tallies_after_a_failed_run():
+    # 2150 collisions of uranium in the metal: lists of 1500 hold the particles
+    # of the one seed's history and not of the other's
+    c, run = _impact("test_metal", (92, 238.03, 1.0))
+    R, V = tg.radial_grid(30, run["Rmin"], run["Rmax"], 100.0)
+    b = Batch([c], R, V, capacity=1500)
+    good, full = 7, run["seed"]
+    (a,) = b.run(good, 0)
+    with pytest.raises(tg.TrekisError, match="capacity"):
+        b.run(full, 0)
+    say("[batch state] a failed run after a good one")
+    with pytest.raises(tg.TrekisError, match="must run before"):
+        b.fetch()
+    b.run(good, 0, with_tallies=False)
+    (f,) = b.fetch()
+    for k in a.arrays:
+        assert np.array_equal(a[k], f[k]), k

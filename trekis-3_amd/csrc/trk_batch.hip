@@ -373,6 +373,7 @@ static int batch_launch(trk_batch *b, uint64_t seed, int64_t first_iter, trk_tal
             b->mc[g][par].iter0 = (uint32_t)first_iter;
         }
     if (!b->exec && batch_capture(b)) return TRK_ERR_DEVICE;
+    b->has_run = false;            // the launch clears the planes: they hold a run's tallies again when it succeeds
     BHIP(b->mixed ? mx::batch_upload(&b->mc[0][0], G, st) : fp64::batch_upload(&b->mc[0][0], G, st));
     BHIP(hipEventRecord(b->ev0, st));
     BHIP(hipGraphLaunch(b->exec, st));
