@@ -42,3 +42,19 @@ def test_no_tallies_after_a_failed_run():
     (f,) = b.fetch()
     for k in a.arrays:
         assert np.array_equal(a[k], f[k]), k
+
+
+def test_round_budget_is_each_groups_own():
+    # oxygen in the oxide (480 collisions, held to the round budget by lists of
+    # 1200) beside lithium in the metal (run on, its rounds may be short): the
+    # oxide's rounds are those it takes alone, whichever material comes first
+    a, _ = _impact("test_metal", (3, 6.94, 0.5))
+    b, run = _impact("test")
+    R, V = tg.radial_grid(30, run["Rmin"], run["Rmax"], 100.0)
+    rounds = []
+    for impacts, first in (([b], 1), ([b, a], 1), ([a, b], 0)):       # the oxide's impact is iteration 1
+        batch = Batch(impacts, R, V, capacity=1200)
+        batch.run(run["seed"], first)
+        rounds.append(batch.timing()[2])
+    say(f"[batch state] rounds alone, first, second: {rounds}")
+    assert rounds[0] == rounds[1] == rounds[2], rounds
