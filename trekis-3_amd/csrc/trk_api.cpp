@@ -255,6 +255,7 @@ int trk_build_tables(trk_ctx *c)
         return set_error(c, TRK_ERR_STATE, "the material context's tables are not built");
     int rc = build_tables(c->hm, c->md, c->ts, c->stream, err, c->base ? &c->base->ts : nullptr, c->mb.oAlpha);
     if (rc) return set_error(c, rc, "table build failed: %s", err.c_str());
+    c->full_cap = 0;
     c->tables_ready = true;
     return 0;
 }
@@ -418,6 +419,7 @@ int trk_tables_finish(trk_ctx *c)
     std::string err;
     const int rc = refresh_derived(c->hm, c->ts, c->stream, err);
     if (rc) return set_error(c, rc, "deriving tables failed: %s", err.c_str());
+    c->full_cap = 0;
     c->tables_dirty = false;
     return 0;
 }

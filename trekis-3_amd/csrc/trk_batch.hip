@@ -77,7 +77,7 @@ struct trk_batch {
     trk::McDev mc[trk::kMaxGroups][2];
     int capacity = 0;
     int block = 768, round_events = 512;
-    bool ion_deep = true;          // ions may take more than round_events collisions in a round
+    bool ion_deep = true;          // ions may take more than round_events collisions in a round (until a list overflows)
     int64_t blocks = 0;
     size_t lds_bytes = 0;
     bool all_staged = false;
@@ -399,7 +399,8 @@ static int batch_launch(trk_batch *b, uint64_t seed, int64_t first_iter, trk_tal
     }
     if (ovf && b->ion_deep) {
         // the same impacts with their ions held to the round budget, which
-        // spreads the pairs over the rounds
+        // spreads the pairs over the rounds; the batch's later runs start so
+        // (its impacts and lists stay the same, see run_core)
         b->ion_deep = false;
         batch_descriptors(b);
         return batch_launch(b, seed, first_iter, outs);
@@ -671,10 +672,16 @@ int trk_batch_tune(trk_batch *b, uint64_t seed, int64_t first_iter)
     b->tune_log.clear();
     double best = 1e300;
     int bb = b->block, bd = b->round_events;
+    // every candidate starts with the ions as the batch has them now, and the
+    // best one's are kept as it was timed with them: a candidate whose lists
+    // overflow holds its own ions to the budget, not those of the next
+    const bool deep = b->ion_deep;
+    bool best_deep = deep;
     for (int blk : blocks)
         for (int dep : depths) {
             b->block = blk;
             b->round_events = dep;
+            b->ion_deep = deep;
             batch_descriptors(b);
             if (batch_shape(b)) continue;
             if (b->exec) { (void)hipGraphExecDestroy(b->exec); b->exec = nullptr; }
@@ -683,10 +690,11 @@ int trk_batch_tune(trk_batch *b, uint64_t seed, int64_t first_iter)
             if (!rc) rc = batch_launch(b, seed, first_iter, nullptr);
             if (rc) return rc;
             b->tune_log.push_back(TuneEntry{blk, dep, b->last_ms});
-            if (b->last_ms < best) { best = b->last_ms; bb = blk; bd = dep; }
+            if (b->last_ms < best) { best = b->last_ms; bb = blk; bd = dep; best_deep = b->ion_deep; }
         }
     b->block = bb;
     b->round_events = bd;
+    b->ion_deep = best_deep;
     batch_descriptors(b);
     if (batch_shape(b)) return TRK_ERR_CAPACITY;
     if (b->exec) { (void)hipGraphExecDestroy(b->exec); b->exec = nullptr; }

@@ -62,6 +62,10 @@ struct trk_ctx {
     // an ion context (trk_ctx_create_ion): the material context whose
     // material arrays and tables this one uses (it must outlive this one)
     const trk_ctx *base = nullptr;
+    // a run whose lists overflowed while its ions ran on beyond the round
+    // budget: capacity of its lists, expected pairs of its ions (0: none)
+    int full_cap = 0;
+    double full_pairs = 0.0;
     // timing of the last run
     double last_transport_s = 0, last_total_s = 0;
     int64_t last_launches = 0;

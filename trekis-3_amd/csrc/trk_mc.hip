@@ -1223,14 +1223,23 @@ static int run_rounds(trk_ctx *c, McState *s, int64_t nmc, uint64_t seed, int64_
 
 // run_rounds, and once more with the ions held to the particles' round budget
 // if a list overflowed while they ran further (nothing has been added to the
-// caller's tallies by then).
+// caller's tallies by then).  Histories that outlast a short round fill the
+// lists whatever the seed (cut-offs of a few eV: the lists overflow at any
+// capacity whose quarter is less than the ion's pairs), so the context keeps
+// the outcome: runs of as many pairs on lists no longer start with their ions
+// held, as batches do after their first overflow, and no run pays twice again.
 static int run_core(trk_ctx *c, McState *s, int64_t nmc, uint64_t seed, int64_t first_iter, const double *Out_R,
                     const double *Out_V, int NR, trk_tallies *out, int64_t B, bool want_spec,
                     const NoAllocBufs *nab = nullptr)
 {
+    const int cap = s->cap[K_EL];
+    const double pairs = (double)B * ion_collisions(c);
+    const bool deep = !(cap <= c->full_cap && pairs >= c->full_pairs);
     bool full = false;
-    const int rc = run_rounds(c, s, nmc, seed, first_iter, Out_R, Out_V, NR, out, B, want_spec, nab, true, &full);
+    const int rc = run_rounds(c, s, nmc, seed, first_iter, Out_R, Out_V, NR, out, B, want_spec, nab, deep, &full);
     if (!rc || !full) return rc;
+    c->full_cap = cap;
+    c->full_pairs = pairs;
     return run_rounds(c, s, nmc, seed, first_iter, Out_R, Out_V, NR, out, B, want_spec, nab, false, &full);
 }
 
