@@ -23,6 +23,7 @@
 //    next) are chosen by trk_batch_tune, which times the candidates on the
 //    batch itself and records every timing.
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <chrono>
 #include <cstdarg>
 #include <cstdio>
@@ -362,11 +363,30 @@ static int batch_capture(trk_batch *b)
 
 static int batch_fetch(trk_batch *b, trk_tallies *const *outs);
 
+// The two stages of the finished tallies, in the first group's hole lists.
+static int batch_reserve(trk_batch *b, trk_tallies *const *outs)
+{
+    size_t values = 0, nodes = 0;
+    for (size_t i = 0; i < b->impacts.size(); ++i) {
+        if (!outs[i]) continue;
+        const trk_ctx *c = b->impacts[i];
+        values = std::max(values, finish_values(c, b->NR, outs[i]));
+        nodes = std::max(nodes, (size_t)c->hm.Nt);
+    }
+    const BatchGroup &g = b->groups[0];
+    for (int k = 0; k < 2; ++k)
+        if (b->fin[k].reserve(values, nodes, g.L[k][K_HO].w, list_bytes((size_t)g.cap[K_HO], 1)))
+            return berr(b, TRK_ERR_DEVICE, "no memory for %zu tally values", values);
+    return 0;
+}
+
 // One replay of the batch graph; host-side tallies only when outs is given.
 static int batch_launch(trk_batch *b, uint64_t seed, int64_t first_iter, trk_tallies *const *outs)
 {
     const int G = (int)b->groups.size();
     hipStream_t st = b->stream;
+    if (outs)
+        if (const int rc = batch_reserve(b, outs)) return rc;
     for (int g = 0; g < G; ++g)
         for (int par = 0; par < 2; ++par) {
             b->mc[g][par].seed = seed;
@@ -658,7 +678,8 @@ int trk_batch_fetch(trk_batch *b, trk_tallies *const *outs)
 {
     if (!b || !outs) return TRK_ERR_ARG;
     if (!b->has_run) return berr(b, TRK_ERR_STATE, "trk_batch_run must run before its tallies are fetched");
-    const int rc = check_outs(b, outs);
+    int rc = check_outs(b, outs);
+    if (!rc) rc = batch_reserve(b, outs);
     return rc ? rc : batch_fetch(b, outs);
 }
 

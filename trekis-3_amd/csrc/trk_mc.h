@@ -281,16 +281,22 @@ bool uses_general_kernel(const HostMat &h);
 // The running sums over time of the tally planes of T, energies as split words
 // (split) or as 128-bit integers.
 hipError_t launch_time_prefix(const Tally &T, int planes, bool split, hipStream_t st);
-// Staging of one plane's finished tallies: device and page-locked host values,
-// kept by the object (context or batch) whose runs use it and grown to the
-// largest plane it was asked for.
+// Staging of one plane's finished tallies: device and page-locked host values.
+// The device values lie in memory that the object (context or batch) has
+// anyway and does not use between a run's transport and the next run, its
+// particle lists; only lists shorter than the results need a buffer of their
+// own.  Reserved before the transport, so that a run which cannot have its
+// memory fails before it has done its work; the host values and the buffer are
+// kept by the object and grown to the largest plane it was asked for.
 struct FinStage {
     double *dev = nullptr, *pin = nullptr;
     unsigned long long *node_sums = nullptr;   // [Nt][4]: lattice energy of the node, the rest of tot_E
     hipEvent_t done = nullptr;                 // the values are in pin
-    size_t n = 0, node_n = 0;
+    size_t n = 0, node_n = 0;                  // what dev and node_sums hold
+    void *own = nullptr;
+    size_t own_bytes = 0, pin_n = 0;
     bool locked = false;                       // pin is page-locked
-    int grow(size_t values, size_t nodes);
+    int reserve(size_t values, size_t nodes, void *room, size_t room_bytes);
     void release();
 };
 // values already on the device that a run adds to another of the caller's arrays
@@ -299,7 +305,9 @@ struct FinExtra {
     double *dst;
     size_t n;
 };
-// One tally plane converted on the device and copied to the stage, and then
+// Values that the finished tallies of a run with these Out_* arrays hold.
+size_t finish_values(const trk_ctx *c, int NR, const trk_tallies *out, const std::vector<FinExtra> *extra = nullptr);
+// One tally plane converted on the device and copied to the reserved stage, and then
 // added into the caller's Out_* arrays (trk_mc.hip).  d_V: Out_V on the device.
 int finish_begin(trk_ctx *c, FinStage &fs, const Tally &T, int plane_index, const double *d_V, int NR,
                  const trk_tallies *out, hipStream_t st, const std::vector<FinExtra> *extra = nullptr);

@@ -685,28 +685,54 @@ static size_t finish_layout(const trk_ctx *c, int NR, const trk_tallies *out, Fi
     return off;
 }
 
-int FinStage::grow(size_t values, size_t nodes)
+size_t finish_values(const trk_ctx *c, int NR, const trk_tallies *out, const std::vector<FinExtra> *extra)
 {
-    if (n >= values && node_n >= nodes) return 0;
-    release();
-    if (hipMalloc((void **)&dev, (values ? values : 1) * sizeof(double)) != hipSuccess ||
-        hipMalloc((void **)&node_sums, (nodes ? nodes : 1) * 4 * sizeof(unsigned long long)) != hipSuccess ||
-        hipEventCreateWithFlags(&done, hipEventDisableTiming) != hipSuccess) {
+    size_t total = finish_layout(c, NR, out, nullptr, nullptr, nullptr);
+    if (extra)
+        for (const FinExtra &x : *extra) total += x.n;
+    return total;
+}
+
+int FinStage::reserve(size_t values, size_t nodes, void *room, size_t room_bytes)
+{
+    n = node_n = 0;
+    if (!done && hipEventCreateWithFlags(&done, hipEventDisableTiming) != hipSuccess) {
         (void)hipGetLastError();
-        release();
+        done = nullptr;
         return 1;
     }
-    // where no memory can be locked, ordinary memory does (slower)
-    const size_t bytes = (values ? values : 1) * sizeof(double);
-    locked = hipHostMalloc((void **)&pin, bytes, hipHostMallocDefault) == hipSuccess;
-    if (!locked) {
-        (void)hipGetLastError();
-        pin = (double *)std::malloc(bytes);
-        if (!pin) {
-            release();
-            return 1;
+    const size_t bytes = values * sizeof(double) + nodes * 4 * sizeof(unsigned long long);
+    if (room_bytes < bytes) {
+        if (own_bytes < bytes) {
+            if (own) (void)hipFree(own);
+            own = nullptr;
+            own_bytes = 0;
+            if (hipMalloc(&own, bytes) != hipSuccess) {
+                (void)hipGetLastError();
+                own = nullptr;
+                return 1;
+            }
+            own_bytes = bytes;
         }
+        room = own;
     }
+    if (pin_n < values || !pin) {
+        // where no memory can be locked, ordinary memory does (slower)
+        const size_t want = (values ? values : 1) * sizeof(double);
+        if (pin && locked) (void)hipHostFree(pin);
+        else std::free(pin);
+        pin = nullptr;
+        pin_n = 0;
+        locked = hipHostMalloc((void **)&pin, want, hipHostMallocDefault) == hipSuccess;
+        if (!locked) {
+            (void)hipGetLastError();
+            pin = (double *)std::malloc(want);
+            if (!pin) return 1;
+        }
+        pin_n = values;
+    }
+    dev = (double *)room;
+    node_sums = (unsigned long long *)(dev + values);
     n = values;
     node_n = nodes;
     return 0;
@@ -714,15 +740,11 @@ int FinStage::grow(size_t values, size_t nodes)
 
 void FinStage::release()
 {
-    if (dev) (void)hipFree(dev);
-    if (node_sums) (void)hipFree(node_sums);
+    if (own) (void)hipFree(own);
     if (pin && locked) (void)hipHostFree(pin);
     else std::free(pin);
     if (done) (void)hipEventDestroy(done);
-    dev = pin = nullptr;
-    node_sums = nullptr;
-    done = nullptr;
-    n = node_n = 0;
+    *this = FinStage{};
 }
 
 // dst += src; runs of zeros (photons of a run without them, nodes before the
@@ -748,11 +770,9 @@ static void add_values(double *dst, const double *src, size_t n)
 int finish_begin(trk_ctx *c, FinStage &fs, const Tally &T, int plane_index, const double *d_V, int NR,
                  const trk_tallies *out, hipStream_t st, const std::vector<FinExtra> *extra)
 {
-    const size_t values = finish_layout(c, NR, out, nullptr, nullptr, nullptr);
-    size_t total = values;
-    if (extra)
-        for (const FinExtra &x : *extra) total += x.n;
-    if (fs.grow(total, (size_t)T.Nt)) return set_error(c, TRK_ERR_DEVICE, "no memory for %zu tally values", total);
+    const size_t values = finish_values(c, NR, out);
+    if (fs.n < finish_values(c, NR, out, extra) || fs.node_n < (size_t)T.Nt)
+        return set_error(c, TRK_ERR_STATE, "the stage of the finished tallies was not reserved");
     FinOut fo{};
     finish_layout(c, NR, out, &fo, fs.dev, nullptr);
     HIPC(launch_finish<false>(c, T, plane_index, d_V, fo, fs.node_sums, st));
@@ -895,6 +915,25 @@ static const void *transport_kernel(bool mixed, bool all, bool general)
                      : (all ? (const void *)fp64::k_transport<true, true> : (const void *)fp64::k_transport<false, true>);
     return mixed ? (all ? (const void *)mx::k_transport<true, false> : (const void *)mx::k_transport<false, false>)
                  : (all ? (const void *)fp64::k_transport<true, false> : (const void *)fp64::k_transport<false, false>);
+}
+
+// The per-iteration accumulators that a run adds to the caller's arrays.
+static std::vector<FinExtra> run_extras(const trk_ctx *c, const McState *s, int NR, const trk_tallies *out, bool want_spec)
+{
+    std::vector<FinExtra> extra;
+    if (!want_spec) return extra;
+    const size_t Nt = (size_t)c->hm.Nt, ND = (size_t)c->hm.m.n_dos;
+    auto add_back = [&](double *dst, const double *src, size_t n) { if (dst) extra.push_back({src, dst, n}); };
+    add_back(out->Out_Ee_vs_E, s->acc_eve, Nt * NR);
+    if (ND > 1) add_back(out->Out_Eh_vs_E, s->acc_ehve, Nt * ND);
+    add_back(out->Out_theta, s->acc_th, (Nt + 1) * 180);
+    add_back(out->Out_theta_h, s->acc_thh, (Nt + 1) * 180);
+    if (c->hm.m.work_function > 0.0) {
+        add_back(out->Out_Ne_Em, s->acc_emn, Nt);
+        add_back(out->Out_E_Em, s->acc_eme, Nt);
+        add_back(out->Out_Ee_vs_E_Em, s->acc_emh, Nt * NR);
+    }
+    return extra;
 }
 
 // The run itself on buffers the caller of this function provides in s (and
@@ -1196,19 +1235,7 @@ static int run_rounds(trk_ctx *c, McState *s, int64_t nmc, uint64_t seed, int64_
         return 0;
     }
     // the finished tallies and the per-iteration accumulators, one transfer
-    std::vector<FinExtra> extra;
-    if (want_spec) {
-        auto add_back = [&](double *dst, const double *src, size_t n) { if (dst) extra.push_back({src, dst, n}); };
-        add_back(out->Out_Ee_vs_E, s->acc_eve, (size_t)Nt * NR);
-        if (ND > 1) add_back(out->Out_Eh_vs_E, s->acc_ehve, (size_t)Nt * ND);
-        add_back(out->Out_theta, s->acc_th, (size_t)(Nt + 1) * 180);
-        add_back(out->Out_theta_h, s->acc_thh, (size_t)(Nt + 1) * 180);
-        if (d.em_W > 0.0) {
-            add_back(out->Out_Ne_Em, s->acc_emn, (size_t)Nt);
-            add_back(out->Out_E_Em, s->acc_eme, (size_t)Nt);
-            add_back(out->Out_Ee_vs_E_Em, s->acc_emh, (size_t)Nt * NR);
-        }
-    }
+    const std::vector<FinExtra> extra = run_extras(c, s, NR, out, want_spec);
     HIPC(hipMemcpyAsync(s->d_V, Out_V, sizeof(double) * NR, hipMemcpyHostToDevice, st));
     int frc = finish_begin(c, s->fin, T, 0, s->d_V, NR, out, st, &extra);
     if (!frc) frc = finish_end(c, s->fin, NR, out, &extra);
@@ -1295,6 +1322,10 @@ int run_mc(trk_ctx *c, int64_t nmc, uint64_t seed, int64_t first_iter, const dou
         }
         if (!s->d_trace_n) HIPC(hipMalloc((void **)&s->d_trace_n, sizeof(unsigned long long)));
     }
+    const std::vector<FinExtra> extra = run_extras(c, s, NR, out, want_spec);
+    const size_t values = finish_values(c, NR, out, &extra);
+    if (s->fin.reserve(values, (size_t)Nt, s->L[0][K_HO].w, list_bytes((size_t)s->cap[K_HO], 1)))
+        return set_error(c, TRK_ERR_DEVICE, "no memory for %zu tally values", values);
     return run_core(c, s, nmc, seed, first_iter, Out_R, Out_V, NR, out, B, want_spec);
 }
 
