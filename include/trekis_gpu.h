@@ -305,7 +305,8 @@ int  trk_batch_error(const trk_batch *b, char *buf, size_t n);
  * first run and replayed after).  outs[i] (may be NULL) receives impact i's
  * tallies as trk_run_mc would add them; the per-iteration normalised ones
  * (Out_Ee_vs_E, Out_Eh_vs_E, Out_theta, Out_theta_h, Out_diff_coeff) must
- * be NULL, and n_events is not filled (see trk_batch_timing). */
+ * be NULL, and n_events is not filled (see trk_batch_timing).  Batches run
+ * from several host threads take turns on a GPU. */
 int  trk_batch_run(trk_batch *b, uint64_t seed, int64_t first_iter, trk_tallies *const *outs);
 /* The tallies of the last trk_batch_run (or tuning run), added into outs as
  * trk_batch_run's outs would be: a caller that runs with outs = NULL keeps

@@ -58,3 +58,29 @@ def test_round_budget_is_each_groups_own():
         rounds.append(batch.timing()[2])
     say(f"[batch state] rounds alone, first, second: {rounds}")
     assert rounds[0] == rounds[1] == rounds[2], rounds
+
+
+def test_batches_on_two_host_threads():
+    import threading
+    impacts = [_impact("test"), _impact("test_metal", (10, 20.18, 0.4))]
+    R, V = tg.radial_grid(30, 1.0, 300.0, 100.0)
+    batches = [Batch([c, c], R, V, capacity=1 << 18) for c, _ in impacts]
+    alone = [b.run(run["seed"], 0) for b, (_, run) in zip(batches, impacts)]
+    got = [[], []]
+
+    def work(i):
+        for _ in range(4):
+            got[i].append(batches[i].run(impacts[i][1]["seed"], 0))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    say("[batch state] two batches, four runs each, side by side")
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for want, runs in zip(alone, got):
+        assert len(runs) == 4
+        for tallies in runs:
+            for x, y in zip(want, tallies):
+                for k in x.arrays:
+                    assert np.array_equal(x[k], y[k]), k

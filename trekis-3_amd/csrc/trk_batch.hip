@@ -30,6 +30,7 @@
 #include <new>
 #include <cstring>
 #include <map>
+#include <mutex>
 #include <string>
 #include <vector>
 #include "trk_mc.h"
@@ -380,6 +381,14 @@ static int batch_reserve(trk_batch *b, trk_tallies *const *outs)
     return 0;
 }
 
+// One batch at a time on a GPU.  The launch reads its descriptors from constant
+// memory that all batches of a path share, and its workgroups must all be
+// resident: a second batch would overwrite the one and could hold back the
+// other.  Batches on other host threads wait here (their tallies are fetched
+// outside).
+constexpr int kMaxDevices = 64;
+static std::mutex g_launch_mu[kMaxDevices];
+
 // One replay of the batch graph; host-side tallies only when outs is given.
 static int batch_launch(trk_batch *b, uint64_t seed, int64_t first_iter, trk_tallies *const *outs)
 {
@@ -394,11 +403,14 @@ static int batch_launch(trk_batch *b, uint64_t seed, int64_t first_iter, trk_tal
         }
     if (!b->exec && batch_capture(b)) return TRK_ERR_DEVICE;
     b->has_run = false;            // the launch clears the planes: they hold a run's tallies again when it succeeds
-    BHIP(b->mixed ? mx::batch_upload(&b->mc[0][0], G, st) : fp64::batch_upload(&b->mc[0][0], G, st));
-    BHIP(hipEventRecord(b->ev0, st));
-    BHIP(hipGraphLaunch(b->exec, st));
-    BHIP(hipEventRecord(b->ev1, st));
-    BHIP(hipEventSynchronize(b->ev1));
+    {
+        std::lock_guard<std::mutex> lk(g_launch_mu[b->device]);
+        BHIP(b->mixed ? mx::batch_upload(&b->mc[0][0], G, st) : fp64::batch_upload(&b->mc[0][0], G, st));
+        BHIP(hipEventRecord(b->ev0, st));
+        BHIP(hipGraphLaunch(b->exec, st));
+        BHIP(hipEventRecord(b->ev1, st));
+        BHIP(hipEventSynchronize(b->ev1));
+    }
     float ms = 0.f;
     BHIP(hipEventElapsedTime(&ms, b->ev0, b->ev1));
     b->last_ms = ms;
@@ -560,6 +572,7 @@ int trk_batch_create(trk_ctx *const *impacts, int32_t n, const double *Out_R, co
     }
     b->mixed = impacts[0]->hm.o.precision == 1;
     b->device = impacts[0]->device;
+    if (b->device < 0 || b->device >= kMaxDevices) return berr(b, TRK_ERR_DEVICE, "device %d out of range", b->device);
     int cur = -1;
     BHIP(hipGetDevice(&cur));
     if (cur != b->device) return berr(b, TRK_ERR_STATE, "the impacts belong to device %d", b->device);
