@@ -508,8 +508,8 @@ def main():
                    "precision": args.precision, "iters_per_step": B,
                    "table_quadrature": "fp32 compensated" if mixed and args.quadrature else "reference fp64",
                    "events": total_ev, "events_by_kind": dict(zip(abi.EVENT_NAMES, ev.tolist())),
-                   "table_build_s": main_leg["t_tables"], "ion_init_kernel_ms": main_leg["ms_shi"],
-                   "ion_init_launches": main_leg["n_shi"],
+                   "table_build_s": main_leg["t_tables"], "ion_kernels_ms": main_leg["ms_shi"],
+                   "ion_kernel_launches": main_leg["n_shi"],
                    "outside_batches_ms_per_step": sum(main_leg["host_ms"]) / len(main_leg["host_ms"]),
                    "vs_fp64": compare},
         # achieved: the algorithmic bytes the kernel moves per launch (state

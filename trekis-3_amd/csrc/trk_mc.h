@@ -122,18 +122,17 @@ struct McDev {
     double *trace; unsigned long long *trace_n; long long trace_cap;
     Tally T;
     Spec S;
-    // used by the mixed path only, and last, so that the offsets of the
-    // fields above stay those the FP64 kernel was tuned with: per-shell
-    // constants of shi_transfer (k_shi_consts), logs of the SHI grid, of
-    // its per-shell paths and of the fused path
+    // the ion's collisions: per-shell constants of its transfer's draw
+    // (k_shi_consts) with the index of its rows by draw (k_shi_buckets), logs
+    // of the SHI grid, of its per-shell paths and of the fused path
     const int *sd_M; const double *sd_c; const int *sd_bk;
     const double *lnES, *ln_LSsh, *ln_shi_path;
-    // batch runs only: the impacts' ions (indexed by iteration - iter0), the
-    // events a particle may take per round, this group's round state
+    // batch runs only: the impacts' ions (indexed by iteration - iter0), this
+    // group's round state
     const IonDev *ions;
     const int *plane_of;        // tally plane of each impact in its group
     uint32_t iter0;
-    int round_events;
+    int round_events;           // events a particle may take per round (round_budget)
     GroupCtl *gctl;
     // emission through the surface Z = 0 (em_W, the work function, > 0): the
     // barrier height, the E1 and gamma of its logistic transmission, and the
@@ -165,8 +164,8 @@ enum { EV_SHI = 0, EV_E_INEL, EV_E_EL, EV_H_INEL, EV_H_EL, EV_AUGER, EV_RAD, EV_
 
 // d.overflow bits: list capacities, the per-particle event limit, NaN state.
 constexpr int kFlagPairs = 1, kFlagPhotons = 2, kFlagEvents = 4, kFlagNaN = 8;
-// Events one particle may process in one launch.  A history needs a few
-// thousand at most; the limit only guarantees that every wave ends.
+// Events one particle may take over all rounds.  A history needs a few
+// thousand at most, an ion 10^5; the limit only guarantees that every run ends.
 constexpr uint32_t kMaxEvents = 1u << 22;
 
 enum { K_EL = 0, K_HO = 1, K_PH = 2, K_ION = 3 };

@@ -307,7 +307,7 @@ hipError_t launch_time_prefix(const Tally &T, int planes, bool split, hipStream_
 struct McState {
     PList L[2][4];            // [ping-pong][electrons, holes, photons, ions]
     int cap[4] = {0, 0, 0, 0};
-    int *d_counts = nullptr;  // [16]: list counts of round A [4], of round B [4], transport cursor
+    int *d_counts = nullptr;  // [16]: list counts of round A [4], of round B [4], transport cursor, ion cursor
     int64_t max_blocks = 0;   // resident transport workgroups on the device
     int ncu = 0, max_lds = 0;
     size_t lds_bytes = 0;     // staged tables per transport workgroup
@@ -514,6 +514,7 @@ void fill_mcdev(const trk_ctx *c, McDev &d)
 
 namespace trk {
 
+// exact integer in units of 2^-40 eV -> double (two roundings at most)
 TRK_DEV double fx_to_double_dev(__int128 v)
 {
     long long hi = (long long)(v >> 40);
@@ -937,8 +938,8 @@ static std::vector<FinExtra> run_extras(const trk_ctx *c, const McState *s, int 
 }
 
 // The run itself on buffers the caller of this function provides in s (and
-// na, for a run without allocation: the tallies are then finished on the
-// device instead of the host).
+// nab, for a run without allocation: the caller's arrays are then added to on
+// the device, otherwise the host adds the finished values).
 // deep: the ions may run further in a round than the other particles; *lists_full
 // is set when a list overflowed with that in use.
 static int run_rounds(trk_ctx *c, McState *s, int64_t nmc, uint64_t seed, int64_t first_iter, const double *Out_R,
@@ -969,9 +970,8 @@ static int run_rounds(trk_ctx *c, McState *s, int64_t nmc, uint64_t seed, int64_
 
     McDev d{};
     fill_mcdev(c, d);
-    // per-shell constants of shi_transfer and the index of its rows by draw,
-    // computed once per table set with the path's own arithmetic (the FP64
-    // path still evaluates the constants in every event, to the same bits)
+    // per-shell constants of the ion's transfer draw and the index of its rows
+    // by draw, computed once per table set with the path's own arithmetic
     if (!c->ts.sd_consts) {
         HIPC(launch_shi_consts(c, ion_view_host(c), mixed, st));
         c->ts.sd_consts = true;
@@ -1218,8 +1218,8 @@ static int run_rounds(trk_ctx *c, McState *s, int64_t nmc, uint64_t seed, int64_
         if (c->trace_n_out) *c->trace_n_out = (int64_t)tn;
     }
 
-    // finalize: replicas summed and time prefix taken on the device (exact
-    // integers); the host converts, scales by Out_V and forms the totals
+    // finalize: replicas summed and time prefix taken (exact integers); the
+    // device then converts, scales by Out_V and forms the totals
     {
         const int64_t ncell = (3 + (int64_t)nsh) * (int64_t)Nt * NR;
         k_replica_sum<<<(unsigned)((ncell + 255) / 256), 256, 0, st>>>(T);
@@ -1463,7 +1463,7 @@ static void carve_state(Carver &cv, McState &s, NoAllocBufs &na, const trk_ctx *
     na.node_sums = cv.take<unsigned long long>((size_t)Nt * 4);
 }
 
-// exact integer in units of 2^-40 eV -> double, as the host finalize converts
+// dst += src
 __global__ void k_add(double *dst, const double *src, int64_t n)
 {
     const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
